@@ -31,11 +31,14 @@ DEVICE_FLAGS = [
 ]
 HOST_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter"]
 
-# (source, object name, flags): exl3_rate.hip once per rate K (0 = any even
-# n), so the rates' kernels compile in parallel.
+# (source, object name, flags): exl3_rate.hip and exl3_rate_gemm.hip once per
+# rate K (0 = any even n, half-integer rates), so the rates' kernels compile
+# in parallel.
 SOURCES = [
     ("exl3_kernels.hip", "exl3_kernels", DEVICE_FLAGS),
     *[("exl3_rate.hip", f"exl3_rate_k{k}", DEVICE_FLAGS + [f"-DEXL3_INST_K={k}"]) for k in range(9)],
+    *[("exl3_rate_gemm.hip", f"exl3_rate_gemm_k{k}", DEVICE_FLAGS + [f"-DEXL3_INST_K={k}"])
+      for k in range(9)],
     ("decoder_ops.hip", "decoder_ops", DEVICE_FLAGS),
     ("exl3_noalloc.hip", "exl3_noalloc", DEVICE_FLAGS),
     ("exl3_host.cpp", "exl3_host", HOST_FLAGS),

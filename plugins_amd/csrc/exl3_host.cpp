@@ -1267,6 +1267,7 @@ exl3_verdict exl3_swiglu(const exl3_weight *gate, const exl3_weight *up, const e
   }
   a.y = out->data;
   a.ydt = xdt;
+  a.aligned = (((uintptr_t)gate->w.data | (uintptr_t)up->w.data | (uintptr_t)down->w.data) & 15) == 0;
   exl3::MoeBank bg{(const uint16_t *)gate->w.data, (const uint16_t *)gate->scales.data,
                    (const uint16_t *)gate->biases.data, pg->f, (int)pg->in, (int)pg->out};
   exl3::MoeBank bu{(const uint16_t *)up->w.data, (const uint16_t *)up->scales.data,
@@ -1396,10 +1397,11 @@ exl3_verdict exl3_swiglu_shared(const exl3_weight *gate, const exl3_weight *up,
   float *r_scores = (float *)((char *)ss->aux + routes);
   a.inds = r_inds;
   a.scores = r_scores;
-  if (exl3::moe_uses_gemm(a, !pg->f.integer_rate(), !pd->f.integer_rate()))
+  if (exl3::moe_prefill_sized(a, !pg->f.integer_rate(), !pd->f.integer_rate()))
     return refuse(EXL3_UNSUPPORTED,
                   "turboexl3_mi355x: the shared expert rides the routed GEMV launches; at "
                   "prefill-sized batches the host runs swiglu and its shared expert's chain");
+  a.verify_rows = true;  // the shared expert rides the decode chain at every other size
   exl3_verdict v = output_for(out, x, hidden, rows, pg->device, s);
   if (v.code != EXL3_OK) return v;
   a.y = out->data;
@@ -1831,6 +1833,7 @@ const char *exl3_swiglu_path(const exl3_weight *gate, const exl3_weight *up,
   a.experts = (int)std::max<int64_t>(pg->experts, 1);
   a.inds = reinterpret_cast<const uint32_t *>(&a);  // routed: any non-null
   a.verify_rows = verify_rows;
+  a.aligned = (((uintptr_t)gate->w.data | (uintptr_t)up->w.data | (uintptr_t)down->w.data) & 15) == 0;
   return exl3::moe_uses_gemm(a, !pg->f.integer_rate(), !pd->f.integer_rate()) ? "routed-gemm"
                                                                               : "routed-gemv";
 }

@@ -1743,12 +1743,18 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_ws_kernel(
                             kpart);
 }
 
-// ==================================================== grouped MoE GEMV
-
-// A work item of the routed MoE: up to GEMV_ROWS slots of one expert.
+// A work item of the routed MoE: slots of one expert.
 struct MoeItem {
   uint32_t expert, start, count, pad;
 };
+
+}  // namespace exl3
+
+#include "exl3_gemm.h"
+
+namespace exl3 {
+
+// ==================================================== grouped MoE GEMV
 
 // Work items of up to 4 slots over splits of up to 256 k-tiles: an item's
 // rows fill at most the rows form's passes (4 rows x 32 blocks), and a
@@ -2045,6 +2051,15 @@ void moe_gemv_go(const Format &f, int pro, dim3 grid, size_t lds, hipStream_t s,
 }
 
 
+// The grouped GEMM over items of up to RDG_ROWS slots.
+template <int K>
+void gemm_rd_grouped_go(const Format &f, unsigned grid, hipStream_t s, const RdGroupArgs &a) {
+  cb_dispatch<K>(f, [&](auto CBC, auto MC) {
+    hipLaunchKernelGGL((gemm_rd_grouped_kernel<K, decltype(CBC)::value, decltype(MC)::value>),
+                       dim3(grid), dim3(64 * RDG_CW), 0, s, a);
+  });
+}
+
 template <int K>
 void gemm_go(const Format &f, dim3 grid, hipStream_t s, const uint32_t *tw, const uint16_t *xp,
              const uint16_t *svh, void *y, int ydt, uint16_t *zout, int M, int in_tiles,
@@ -2084,6 +2099,8 @@ void gemm_frac_go(const Format &f, dim3 grid, hipStream_t s, const uint32_t *tw,
 #define EXL3_GEMM_GROUPED_GO(KK)                                                             \
   void gemm_grouped_go<KK>(const Format &, dim3, hipStream_t, const uint32_t *, const uint16_t *, \
                            const uint16_t *, void *, int, int, int, const GemmGroup &)
+#define EXL3_GEMM_RD_GROUPED_GO(KK) \
+  void gemm_rd_grouped_go<KK>(const Format &, unsigned, hipStream_t, const RdGroupArgs &)
 #define EXL3_GEMM_GO(KK)                                                                    \
   void gemm_go<KK>(const Format &, dim3, hipStream_t, const uint32_t *, const uint16_t *, \
                    const uint16_t *, void *, int, uint16_t *, int, int, int, float *)
@@ -2108,20 +2125,28 @@ EXL3_EXTERN_RATE(8)
 #undef EXL3_EXTERN_RATE
 extern template EXL3_GEMM_GO(1);
 extern template EXL3_GEMM_GROUPED_GO(1);
+extern template EXL3_GEMM_RD_GROUPED_GO(1);
 extern template EXL3_GEMM_GO(2);
 extern template EXL3_GEMM_GROUPED_GO(2);
+extern template EXL3_GEMM_RD_GROUPED_GO(2);
 extern template EXL3_GEMM_GO(3);
 extern template EXL3_GEMM_GROUPED_GO(3);
+extern template EXL3_GEMM_RD_GROUPED_GO(3);
 extern template EXL3_GEMM_GO(4);
 extern template EXL3_GEMM_GROUPED_GO(4);
+extern template EXL3_GEMM_RD_GROUPED_GO(4);
 extern template EXL3_GEMM_GO(5);
 extern template EXL3_GEMM_GROUPED_GO(5);
+extern template EXL3_GEMM_RD_GROUPED_GO(5);
 extern template EXL3_GEMM_GO(6);
 extern template EXL3_GEMM_GROUPED_GO(6);
+extern template EXL3_GEMM_RD_GROUPED_GO(6);
 extern template EXL3_GEMM_GO(7);
 extern template EXL3_GEMM_GROUPED_GO(7);
+extern template EXL3_GEMM_RD_GROUPED_GO(7);
 extern template EXL3_GEMM_GO(8);
 extern template EXL3_GEMM_GROUPED_GO(8);
+extern template EXL3_GEMM_RD_GROUPED_GO(8);
 extern template EXL3_GEMM_FRAC_GO(3);
 extern template EXL3_GEMM_FRAC_GO(5);
 #endif

@@ -259,11 +259,15 @@ struct MoeArgs {
   // the decode chain (grouped GEMV items) at any row count
   // (exl3_swiglu_opts.verify_rows)
   bool verify_rows;
+  bool aligned = true;  // the banks' trellises are 16-byte aligned
 };
-// Whether a routed call takes the grouped GEMM (prefill-sized expert
-// batches: at least 32 slots per expert on average, integer rates, and not
-// verify_rows) rather than the grouped GEMV's items of up to 4 slots.
+// Whether a routed call takes the grouped GEMM (more than 16 slots per
+// expert on average, integer rates, aligned, and not verify_rows) rather
+// than the grouped GEMV's items of up to 4 slots.
 bool moe_uses_gemm(const MoeArgs &a, bool gu_generic, bool d_generic);
+// Whether a call counts as prefill-sized (32 slots per expert on average):
+// swiglu_shared refuses such calls.
+bool moe_prefill_sized(const MoeArgs &a, bool gu_generic, bool d_generic);
 // Staging bytes for a call, and (in *partial_floats) the partial-sum slots
 // of its Scratch.
 size_t moe_scratch_bytes(const MoeArgs &a, bool gu_generic, bool d_generic,

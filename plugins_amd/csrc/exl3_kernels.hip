@@ -1159,8 +1159,9 @@ struct MoeLayout {
   size_t sorted, items, n_items, g, u, xd, d, xg, xu, total;
   size_t partial_floats;  // slots in the separate slot buffer: gate, up, down
   int slots, max_items, ks_gu, ks_d, tps_gu, tps_d;
-  bool gemm;  // prefill-sized expert batches: grouped GEMMs over 256-slot items
+  bool gemm;  // larger expert batches: grouped GEMMs over items of up to RDG_ROWS slots
   bool direct;  // one row, routes given: every slot its own one-row item
+  int item_rows;  // slots an item holds at most
 };
 
 // Down GEMV launches of at most this many workgroups take the mid step in
@@ -1169,8 +1170,15 @@ struct MoeLayout {
 constexpr size_t MOE_FUSED_MID_MAX_WG = 2048;
 
 // Grouped GEMMs when the slots average at least this many per expert (and
-// every rate is an integer rate); below, the routed GEMV items.
-constexpr int MOE_GEMM_SLOTS_PER_EXPERT = 32;
+// every rate is an integer rate); below, the routed GEMV items, which decode
+// an expert's weights once per 4 slots: 16 experts of 4096 x 2048 at K = 3,
+// 17 / 24 / 32 slots each, 250 / 325 / 470 us a call through the items
+// against 115 / 118 / 122 through the GEMM.  (Calls of up to 16 slots an
+// expert keep the decode chain's sums.)
+constexpr int MOE_GEMM_SLOTS_PER_EXPERT = 17;
+// ... and the average from which a call counts as prefill-sized: swiglu_shared
+// refuses such batches.
+constexpr int MOE_PREFILL_SLOTS_PER_EXPERT = 32;
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
@@ -1178,8 +1186,13 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 bool moe_uses_gemm(const MoeArgs &a, bool gu_generic, bool d_generic) {
   const long slots = (long)a.rows * a.topk;
-  return !gu_generic && !d_generic && a.inds != nullptr && !a.verify_rows &&
+  return !gu_generic && !d_generic && a.inds != nullptr && !a.verify_rows && a.aligned &&
          slots >= (long)MOE_GEMM_SLOTS_PER_EXPERT * a.experts;
+}
+
+bool moe_prefill_sized(const MoeArgs &a, bool gu_generic, bool d_generic) {
+  return !gu_generic && !d_generic &&
+         (long)a.rows * a.topk >= (long)MOE_PREFILL_SLOTS_PER_EXPERT * a.experts;
 }
 
 namespace {
@@ -1218,7 +1231,8 @@ MoeLayout moe_layout(const MoeArgs &a, bool generic_gu, bool generic_d) {
   // the routes directly (no route launch; a row's routes name distinct
   // experts, and a repeated one would only be read twice)
   L.direct = !L.gemm && a.rows == 1 && a.inds != nullptr;
-  const int item_rows = L.gemm ? GM_BM : MOE_ITEM_ROWS;
+  const int item_rows = L.item_rows =
+      L.gemm ? RDG_ROWS : MOE_ITEM_ROWS;
   L.max_items = std::min(a.experts, slots) + (slots + item_rows - 1) / item_rows;
   const int groups = std::max(1, std::min(a.experts, slots));
   moe_plan(a.hidden, a.inter, 2 * groups, L.direct, &L.ks_gu, &L.tps_gu);
@@ -1387,26 +1401,40 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
     // prefill-sized expert batches: per-slot prepared rows, grouped GEMMs
     // gate and up, the mid step, grouped GEMM down, the weighted sum
     hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(MOE_ROUTE_THREADS), 0, s, a.inds, L.slots,
-                       a.experts, sorted, items, n_items, (uint32_t)GM_BM);
+                       a.experts, sorted, items, n_items, (uint32_t)L.item_rows);
     uint16_t *xg = (uint16_t *)(base + L.xg), *xu = (uint16_t *)(base + L.xu);
     const int nblk = a.hidden / 128;
     hipLaunchKernelGGL(moe_prep_kernel, dim3((nblk + 3) / 4, L.slots), dim3(256), 0, s, a.x,
                        a.xdt, a.inds, a.experts, a.topk, gate.suh, up.suh, xg, xu, a.hidden, nblk);
-    auto grouped = [&](const MoeBank &b, const uint16_t *xp, uint16_t *yo) {
-      GemmGroup gg{sorted, items, n_items, (size_t)(b.in / 16) * (b.out / 16) * (b.f.n / 2)};
-      const dim3 grid(b.out / 128, L.max_items);
-      const uint32_t *tw = reinterpret_cast<const uint32_t *>(b.trellis);
-      rate_dispatch(b.f.n / 16, [&](auto KC) {
+    auto grouped = [&](const MoeBank *const *b, const uint16_t *const *xp, uint16_t *const *yo,
+                       int nw) {
+      RdGroupArgs r{};
+      r.nw = nw;
+      r.ydt = OUT_F16;
+      r.in_tiles = b[0]->in / 16;
+      r.dec = b[0]->f.dec();
+      r.sorted = sorted;
+      r.items = items;
+      r.n_items = n_items;
+      for (int i = 0; i < nw; ++i) {
+        r.w[i] = RdGroupWeight{reinterpret_cast<const uint32_t *>(b[i]->trellis), xp[i], b[i]->svh,
+                               yo[i], (size_t)(b[i]->in / 16) * (b[i]->out / 16) * (b[i]->f.n / 2),
+                               b[i]->out / 16, r.ct};
+        r.ct += (b[i]->out + 64 * RDG_CW - 1) / (64 * RDG_CW);
+      }
+      const unsigned grid = (unsigned)r.ct * ((L.max_items + 7) / 8 * 8);
+      rate_dispatch(b[0]->f.n / 16, [&](auto KC) {
         constexpr int K = decltype(KC)::value;
-        if constexpr (K > 0)
-          gemm_grouped_go<K>(b.f, grid, s, tw, xp, b.svh, yo, OUT_F16, b.in / 16, b.out / 16, gg);
+        if constexpr (K > 0) gemm_rd_grouped_go<K>(b[0]->f, grid, s, r);
       });
     };
-    grouped(gate, xg, g);
-    grouped(up, xu, u);
+    const MoeBank *const gub[2] = {&gate, &up}, *const db[1] = {&down};
+    const uint16_t *const gux[2] = {xg, xu}, *const dx[1] = {xd};
+    uint16_t *const guy[2] = {g, u}, *const dy[1] = {d};
+    grouped(gub, gux, guy, 2);
     hipLaunchKernelGGL(moe_mid_kernel, dim3(a.inter / 128, L.slots), dim3(64), 0, s, g, u, a.inds,
                        a.experts, down.suh, xd, a.inter, a.limit, -1, nullptr);
-    grouped(down, xd, d);
+    grouped(db, dx, dy, 1);
     hipLaunchKernelGGL(moe_combine_kernel, dim3((a.hidden + 255) / 256, a.rows), dim3(256), 0, s,
                        d, a.inds, a.scores, a.sdt, a.topk, a.experts, a.hidden, a.y, a.ydt);
     return hipGetLastError();

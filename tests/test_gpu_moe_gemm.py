@@ -1,0 +1,48 @@
+"""The routed experts' grouped GEMM at the edges of its tiles: item sizes on
+both sides of a row block (32), of the tile forms (64, 128) and of an item
+(128), a column tile that is half empty (widths of an odd number of 128-column
+groups), every codebook form's operand path and rates on both sides of the
+word stages' limits, against the oracle's composition."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle import oracle as O  # noqa: E402
+from plugins_amd import exl3 as X  # noqa: E402
+from tests import _synth as S  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _bank(rng, experts, in_f, out_f, n, codebook):
+    t, u, v = S.linear(rng, in_f, out_f, n, experts=experts)
+    d = [torch.from_numpy(t.view(np.int16)).to(DEV), torch.from_numpy(u.view(np.float16)).to(DEV),
+         torch.from_numpy(v.view(np.float16)).to(DEV)]
+    return (t, u, v), X.wrap(*d, codebook=codebook)
+
+
+@pytest.mark.parametrize("counts", [(1, 31, 32, 33, 40), (63, 64, 65, 0, 20), (127, 128, 129, 1, 1),
+                                    (260, 5, 96, 97, 17)])
+@pytest.mark.parametrize("n,hidden,inter", [(48, 384, 640), (16, 128, 256), (112, 256, 384),
+                                            (128, 512, 128)])
+def test_grouped_gemm_item_edges(counts, n, hidden, inter):
+    rng = np.random.default_rng(sum(counts) + n)
+    E = len(counts)
+    inds = np.repeat(np.arange(E, dtype=np.int32), counts)
+    rng.shuffle(inds)
+    rows = inds.size
+    inds = inds.reshape(rows, 1)
+    scores = rng.uniform(0.2, 1.0, (rows, 1)).astype(np.float32)
+    gn, g = _bank(rng, E, hidden, inter, n, "mul1")
+    un, u = _bank(rng, E, hidden, inter, n, "mul1")
+    dn, d = _bank(rng, E, inter, hidden, n, "mul1")
+    x = S.activations(rng, rows, hidden)
+    assert X.swiglu_path(g, u, d, rows, 1) == "routed-gemm"
+    y = X.swiglu(g, u, d, torch.from_numpy(x).to(DEV), torch.from_numpy(inds).to(DEV),
+                 torch.from_numpy(scores).to(DEV)).float().cpu().numpy()
+    want = O.moe_swiglu(x.astype(np.float32), gn, un, dn, inds, scores, hidden, inter, n)
+    # the repository's bar: three f16 rounding points a linear, 2^-11 each
+    assert S.rel_fro(y, want) < 1e-3
+    assert S.row_rel(y, want).max() < 3e-3
