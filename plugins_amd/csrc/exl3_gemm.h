@@ -514,18 +514,16 @@ constexpr int RDG_CW = 4, RDG_ROWS = 128;
 // Routed work items: workgroup (column tile, item), the item up to RDG_ROWS
 // slots of one expert (sorted[start ..]); activation rows gathered by slot (xp
 // holds one prepared row per slot), expert e's words and svh, outputs
-// scattered to the slots' rows.  One k-part, so four-wave workgroups, two a CU
-// by registers.  Up to two weights (gate and up) side by side in the column
-// tiles.
+// scattered to the slots' rows.  One k-part, so four-wave workgroups.  Up to
+// two weights (gate and up) side by side in the column tiles.  A launch's
+// items hold up to 32 MRMAX slots (2: four workgroups a CU, 4: two).
 //
 // Against a workgroup of 256 rows x 128 columns whose eight decode waves fill
 // LDS for eight MFMA waves (what ran before), on 256 experts of 7168 x 2048 at
 // K = 3 with 32 slots each (moe layer of 1024 tokens): gate + up 3380 -> 1220
 // us, down 1990 -> 665 us, which is 2.3 and 2.1 TB/s of packed words; 16
 // experts of 4096 x 2048 with 128 / 1024 slots each, the whole call, 273 ->
-// 253 and 1478 -> 1373 us.  Items of up to 64 slots (half the accumulators,
-// twice the workgroups a CU) measured the same at 32 slots an expert and
-// 6-16 % slower from 64 on.
+// 253 and 1478 -> 1373 us.
 struct RdGroupWeight {
   const uint32_t *tw;
   const uint16_t *xp;   // [slots][in]
@@ -580,10 +578,10 @@ __device__ __forceinline__ void rd_group_tile(const RdGroupArgs &a, const RdGrou
                     nullptr, W.svh + (size_t)item.expert * out, W.y, a.ydt, nullptr);
 }
 
-template <int K, int CB, bool MASKED>
-__global__ __launch_bounds__(64 * RDG_CW, (rd_waves<K, 0, RDG_ROWS / 32, RDG_CW, 1>())) void
+template <int K, int CB, bool MASKED, int MRMAX>
+__global__ __launch_bounds__(64 * RDG_CW, (rd_waves<K, 0, MRMAX, RDG_CW, 1>())) void
 gemm_rd_grouped_kernel(RdGroupArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[rd_lds_bytes<K, 0, RDG_ROWS / 32, RDG_CW, 1>()];
+  __shared__ __attribute__((aligned(16))) char smem[rd_lds_bytes<K, 0, MRMAX, RDG_CW, 1>()];
   // Workgroup n runs on XCD n % 8: an item's column tiles go to one XCD, whose
   // L2 then holds the item's activations.  (Only the speed depends on this;
   // the grid holds a multiple of 8 items, some past the last.)
@@ -595,9 +593,13 @@ gemm_rd_grouped_kernel(RdGroupArgs a) {
   const RdGroupWeight &W = a.w[wi];
   const int ct = gx - W.ct0;
   // the row blocks that hold the item (1, 2 or 4)
-  if ((int)item.count > 64)
-    rd_group_tile<K, CB, MASKED, 4, 0>(a, W, ct, item, smem);
-  else if ((int)item.count > 32)
+  if constexpr (MRMAX > 2) {
+    if ((int)item.count > 64) {
+      rd_group_tile<K, CB, MASKED, 4, 0>(a, W, ct, item, smem);
+      return;
+    }
+  }
+  if ((int)item.count > 32)
     rd_group_tile<K, CB, MASKED, 2, 0>(a, W, ct, item, smem);
   else
     rd_group_tile<K, CB, MASKED, 1, 0>(a, W, ct, item, smem);

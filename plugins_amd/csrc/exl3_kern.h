@@ -2051,12 +2051,20 @@ void moe_gemv_go(const Format &f, int pro, dim3 grid, size_t lds, hipStream_t s,
 }
 
 
-// The grouped GEMM over items of up to RDG_ROWS slots.
+// The grouped GEMM over items of up to item_rows slots (RDG_ROWS or half).
 template <int K>
-void gemm_rd_grouped_go(const Format &f, unsigned grid, hipStream_t s, const RdGroupArgs &a) {
+void gemm_rd_grouped_go(const Format &f, int item_rows, unsigned grid, hipStream_t s,
+                        const RdGroupArgs &a) {
   cb_dispatch<K>(f, [&](auto CBC, auto MC) {
-    hipLaunchKernelGGL((gemm_rd_grouped_kernel<K, decltype(CBC)::value, decltype(MC)::value>),
-                       dim3(grid), dim3(64 * RDG_CW), 0, s, a);
+    constexpr int CB = decltype(CBC)::value;
+    constexpr bool M = decltype(MC)::value;
+    const dim3 blk(64 * RDG_CW);
+    if (item_rows < RDG_ROWS)
+      hipLaunchKernelGGL((gemm_rd_grouped_kernel<K, CB, M, RDG_ROWS / 64>), dim3(grid), blk, 0, s,
+                         a);
+    else
+      hipLaunchKernelGGL((gemm_rd_grouped_kernel<K, CB, M, RDG_ROWS / 32>), dim3(grid), blk, 0, s,
+                         a);
   });
 }
 
@@ -2100,7 +2108,7 @@ void gemm_frac_go(const Format &f, dim3 grid, hipStream_t s, const uint32_t *tw,
   void gemm_grouped_go<KK>(const Format &, dim3, hipStream_t, const uint32_t *, const uint16_t *, \
                            const uint16_t *, void *, int, int, int, const GemmGroup &)
 #define EXL3_GEMM_RD_GROUPED_GO(KK) \
-  void gemm_rd_grouped_go<KK>(const Format &, unsigned, hipStream_t, const RdGroupArgs &)
+  void gemm_rd_grouped_go<KK>(const Format &, int, unsigned, hipStream_t, const RdGroupArgs &)
 #define EXL3_GEMM_GO(KK)                                                                    \
   void gemm_go<KK>(const Format &, dim3, hipStream_t, const uint32_t *, const uint16_t *, \
                    const uint16_t *, void *, int, uint16_t *, int, int, int, float *)

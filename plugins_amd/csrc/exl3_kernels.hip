@@ -907,9 +907,22 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_route_kernel(
   if (t == 0) *n_items = total;
 }
 
+// Eight consecutive elements at element i of a 2-byte array as dwords; wide:
+// the array is 16-byte aligned (i a multiple of 8).
+__device__ __forceinline__ uint4 load8_16(const uint16_t *p, size_t i, bool wide) {
+  if (wide) return *reinterpret_cast<const uint4 *>(p + i);
+  uint32_t w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = (uint32_t)p[i + 2 * e] | ((uint32_t)p[i + 2 * e + 1] << 16);
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // The grouped GEMM's gate and up inputs: slot s's row x[s / topk] prepared
-// with expert e = inds[s]'s suh of each (as prepare_kernel: f16(x) * suh,
-// Hadamard-128, * 1/sqrt(128), f16), one wave per 128-block.
+// with expert e = inds[s]'s suh of each (as prepare8_kernel: f16(x) * suh,
+// Hadamard-128, * 1/sqrt(128), f16), 16 lanes a 128-block of the flattened
+// [slots][in / 128].  Bound by its writes (2 x slots x in f16): 16-byte
+// accesses, 1024 tokens x top 8 of 7168: 157 -> 88 us against a wave per
+// block and 4-byte accesses.  wide: x and both suh are 16-byte aligned.
 __global__ __launch_bounds__(256) void moe_prep_kernel(const void *__restrict__ x, int xdt,
                                                        const uint32_t *__restrict__ inds,
                                                        int experts, int topk,
@@ -917,89 +930,154 @@ __global__ __launch_bounds__(256) void moe_prep_kernel(const void *__restrict__ 
                                                        const uint16_t *__restrict__ suh_u,
                                                        uint16_t *__restrict__ xg,
                                                        uint16_t *__restrict__ xu, int in,
-                                                       int nblk) {
-  const int lane = threadIdx.x & 63;
-  const int blk = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (blk >= nblk) return;  // whole waves
-  const size_t slot = blockIdx.y;
-  const uint32_t e = inds[slot];
-  if (e >= (uint32_t)experts) return;
-  const int k = blk * 128 + 2 * lane;
-  const size_t xrow = (slot / (size_t)topk) * in;
-  const float x0 = h2f(f2h(load_act(x, xrow + k, xdt))), x1 = h2f(f2h(load_act(x, xrow + k + 1, xdt)));
-  const uint16_t *const su[2] = {suh_g + (size_t)e * in, suh_u + (size_t)e * in};
-  uint16_t *const dst[2] = {xg, xu};
+                                                       uint32_t nblocks, int wide) {
+  const int j = threadIdx.x & 15;
+  const uint32_t gb0 = blockIdx.x * 16u + (threadIdx.x >> 4);
+  const uint32_t gb = min(gb0, nblocks - 1);  // past the last: redone, not stored
+  const uint32_t nblk = (uint32_t)in / 128u;
+  const uint32_t slot = gb / nblk;
+  const int k = (int)(gb - slot * nblk) * 128 + 8 * j;
+  const uint32_t e0 = inds[slot];
+  const bool valid = gb0 < nblocks && e0 < (uint32_t)experts;
+  const size_t e = valid ? e0 : 0;  // (all lanes take part in the exchanges)
+  const size_t xo = (size_t)(slot / (uint32_t)topk) * in + k;
+  uint32_t h[4];
+  if (xdt == OUT_F32) {
 #pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    const uint32_t sv = *reinterpret_cast<const uint32_t *>(su[w] + k);
-    float v0 = x0 * h2f((uint16_t)(sv & 0xFFFFu)), v1 = x1 * h2f((uint16_t)(sv >> 16));
-    had128_pair(v0, v1, lane);
-    *reinterpret_cast<uint32_t *>(dst[w] + slot * in + k) =
-        (uint32_t)f2h(v0 * HAD_SCALE) | ((uint32_t)f2h(v1 * HAD_SCALE) << 16);
+    for (int i = 0; i < 4; ++i)
+      h[i] = (uint32_t)f2h(((const float *)x)[xo + 2 * i]) |
+             ((uint32_t)f2h(((const float *)x)[xo + 2 * i + 1]) << 16);
+  } else {
+    const uint4 w = load8_16((const uint16_t *)x, xo, wide != 0);
+    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      h[i] = xdt == OUT_F16 ? ws[i]
+                            : (uint32_t)f2h(bits<float>(ws[i] << 16)) |
+                                  ((uint32_t)f2h(bits<float>(ws[i] & 0xFFFF0000u)) << 16);
+  }
+  const uint4 g = prep_block8(h, load8_16(suh_g, e * in + k, wide != 0), j);
+  const uint4 u = prep_block8(h, load8_16(suh_u, e * in + k, wide != 0), j);
+  if (valid) {
+    *reinterpret_cast<uint4 *>(xg + (size_t)slot * in + k) = g;
+    *reinterpret_cast<uint4 *>(xu + (size_t)slot * in + k) = u;
   }
 }
 
 // The mid step: h = silu(g) * u (clamped when limit > 0), then down's
-// prepare with suh_d[e] (the shared expert's, sh_suh_d, for e == shared).
+// prepare with suh_d[e] (the shared expert's, sh_suh_d, for e == shared), 16
+// lanes a 128-block of the flattened [slots][inter / 128] (16-byte accesses:
+// 8192 slots of 2048, 48 -> 33 us against a wave a block and 2-byte ones).
 // A down GEMV launch of few workgroups forms the same values, bit for bit,
-// in its SwiGLU prologue instead.
-__global__ __launch_bounds__(64) void moe_mid_kernel(const uint16_t *__restrict__ g,
-                                                     const uint16_t *__restrict__ u,
-                                                     const uint32_t *__restrict__ inds, int experts,
-                                                     const uint16_t *__restrict__ suh_d,
-                                                     uint16_t *__restrict__ xd, int inter,
-                                                     float limit, int shared,
-                                                     const uint16_t *__restrict__ sh_suh_d) {
-  const int lane = threadIdx.x;
-  const size_t slot = blockIdx.y;
-  const uint32_t e = inds ? inds[slot] : 0u;
-  if (e >= (uint32_t)experts) return;
-  const uint16_t *sud = (int)e == shared ? sh_suh_d : suh_d + (size_t)e * inter;
-  const int i0 = blockIdx.x * 128 + lane;
-  float v[2];
+// in its SwiGLU prologue instead.  wide: the suh arrays are 16-byte aligned.
+__global__ __launch_bounds__(256) void moe_mid_kernel(const uint16_t *__restrict__ g,
+                                                      const uint16_t *__restrict__ u,
+                                                      const uint32_t *__restrict__ inds,
+                                                      int experts,
+                                                      const uint16_t *__restrict__ suh_d,
+                                                      uint16_t *__restrict__ xd, int inter,
+                                                      float limit, int shared,
+                                                      const uint16_t *__restrict__ sh_suh_d,
+                                                      uint32_t nblocks, int wide) {
+  const int j = threadIdx.x & 15;
+  const uint32_t gb0 = blockIdx.x * 16u + (threadIdx.x >> 4);
+  const uint32_t gb = min(gb0, nblocks - 1);
+  const uint32_t nblk = (uint32_t)inter / 128u;
+  const uint32_t slot = gb / nblk;
+  const int k = (int)(gb - slot * nblk) * 128 + 8 * j;
+  const uint32_t e0 = inds ? inds[slot] : 0u;
+  const bool valid = gb0 < nblocks && e0 < (uint32_t)experts;
+  const bool sh = valid && (int)e0 == shared;
+  const uint16_t *sud = sh ? sh_suh_d : suh_d + (valid ? (size_t)e0 * inter : 0);
+  const size_t off = (size_t)slot * inter + k;
+  const uint4 gv = *reinterpret_cast<const uint4 *>(g + off);
+  const uint4 uv = *reinterpret_cast<const uint4 *>(u + off);
+  const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
+  uint32_t h[4];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int i = i0 + 64 * j;
-    float gv = h2f(g[slot * inter + i]), uv = h2f(u[slot * inter + i]);
-    if (limit > 0.0f) swiglu_clamp(gv, uv, limit);
-    const float h = f32_value(gv / (1.0f + expf(-gv))) * uv;
-    v[j] = h2f(f2h(h)) * h2f(sud[i]);
-  }
-#pragma unroll
-  for (int bit = 1; bit <= 32; bit <<= 1) {
-    const float p0 = xor_lanes(v[0], bit), p1 = xor_lanes(v[1], bit);
-    const float sg = (lane & bit) == 0 ? 1.0f : -1.0f;
-    v[0] = butterfly(sg, v[0], p0);
-    v[1] = butterfly(sg, v[1], p1);
-  }
-  const float a = v[0] + v[1], b = v[0] - v[1];
-  xd[slot * inter + i0] = f2h(a * HAD_SCALE);
-  xd[slot * inter + i0 + 64] = f2h(b * HAD_SCALE);
+  for (int i = 0; i < 4; ++i)
+    h[i] = (uint32_t)f2h(swiglu1((uint16_t)(gw[i] & 0xFFFFu), (uint16_t)(uw[i] & 0xFFFFu), limit)) |
+           ((uint32_t)f2h(swiglu1((uint16_t)(gw[i] >> 16), (uint16_t)(uw[i] >> 16), limit)) << 16);
+  const uint4 o = prep_block8(h, load8_16(sud, k, wide != 0), j);
+  if (valid) *reinterpret_cast<uint4 *>(xd + off) = o;
 }
 
-// y[row] = sum_k score * d[slot] (f32, k order), in the output dtype.
-__global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t *__restrict__ d,
+void launch_moe_mid(const uint16_t *g, const uint16_t *u, const uint32_t *inds, int experts,
+                    const uint16_t *suh_d, uint16_t *xd, int slots, int inter, float limit,
+                    int shared, const uint16_t *sh_suh_d, hipStream_t s) {
+  const uint32_t nblocks = (uint32_t)slots * (uint32_t)(inter / 128);
+  const int wide = (((uintptr_t)suh_d | (uintptr_t)sh_suh_d) & 15) == 0;
+  hipLaunchKernelGGL(moe_mid_kernel, dim3((nblocks + 15) / 16), dim3(256), 0, s, g, u, inds,
+                     experts, suh_d, xd, inter, limit, shared, sh_suh_d, nblocks, wide);
+}
+
+// y[row] = sum_k score * d[slot] (f32, k order), in the output dtype: eight
+// columns a thread, eight slots' loads in flight before their sums (1024 rows
+// x top 8 of 7168: 84 -> 24 us against a column a thread).  wide: y is 16-byte
+// aligned.
+__global__ __launch_bounds__(128) void moe_combine_kernel(const uint16_t *__restrict__ d,
                                                           const uint32_t *__restrict__ inds,
                                                           const void *__restrict__ scores, int sdt,
                                                           int topk, int experts, int hidden,
-                                                          void *__restrict__ y, int ydt) {
+                                                          void *__restrict__ y, int ydt, int wide) {
   const size_t row = blockIdx.y;
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int i = 8 * (blockIdx.x * 128 + threadIdx.x);
   if (i >= hidden) return;
-  float acc = 0.0f;
-  for (int k = 0; k < topk; ++k) {
-    const size_t slot = row * topk + k;
-    const uint32_t e = inds ? inds[slot] : 0u;
-    if (e >= (uint32_t)experts) continue;
-    const float w = scores ? load_act(scores, slot, sdt) : 1.0f;
-    acc = acc + f32_value(w * h2f(d[slot * hidden + i]));
+  float acc[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) acc[c] = 0.0f;
+  for (int k0 = 0; k0 < topk; k0 += 8) {
+    uint4 v[8];
+    float w[8];
+    bool on[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const size_t slot = row * topk + min(k0 + q, topk - 1);
+      on[q] = k0 + q < topk && (inds ? inds[slot] : 0u) < (uint32_t)experts;
+      w[q] = scores ? load_act(scores, slot, sdt) : 1.0f;
+      if (on[q]) v[q] = *reinterpret_cast<const uint4 *>(d + slot * hidden + i);
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (!on[q]) continue;
+      const uint32_t ws[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        acc[2 * c] = acc[2 * c] + f32_value(w[q] * h2f((uint16_t)(ws[c] & 0xFFFFu)));
+        acc[2 * c + 1] = acc[2 * c + 1] + f32_value(w[q] * h2f((uint16_t)(ws[c] >> 16)));
+      }
+    }
   }
-  if (ydt == OUT_F16)
-    ((uint16_t *)y)[row * hidden + i] = f2h(acc);
-  else if (ydt == OUT_BF16)
-    ((uint16_t *)y)[row * hidden + i] = f2bf(acc);
-  else
-    ((float *)y)[row * hidden + i] = acc;
+  const size_t o = row * hidden + i;
+  if (ydt == OUT_F32) {
+    float *p = (float *)y + o;
+    if (wide) {
+      *reinterpret_cast<float4 *>(p) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      *reinterpret_cast<float4 *>(p + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) p[c] = acc[c];
+    }
+    return;
+  }
+  uint16_t r[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) r[c] = ydt == OUT_F16 ? f2h(acc[c]) : f2bf(acc[c]);
+  uint16_t *p = (uint16_t *)y + o;
+  if (wide) {
+    *reinterpret_cast<uint4 *>(p) =
+        make_uint4((uint32_t)r[0] | ((uint32_t)r[1] << 16), (uint32_t)r[2] | ((uint32_t)r[3] << 16),
+                   (uint32_t)r[4] | ((uint32_t)r[5] << 16), (uint32_t)r[6] | ((uint32_t)r[7] << 16));
+  } else {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) p[c] = r[c];
+  }
+}
+
+void launch_moe_combine(const MoeArgs &a, const uint16_t *d, hipStream_t s) {
+  hipLaunchKernelGGL(moe_combine_kernel, dim3((a.hidden / 8 + 127) / 128, a.rows), dim3(128), 0, s,
+                     d, a.inds, a.scores, a.sdt, a.topk, a.experts, a.hidden, a.y, a.ydt,
+                     (int)(((uintptr_t)a.y & 15) == 0));
 }
 
 // The routes of a swiglu with a shared expert (launch_moe_shared_route): one
@@ -1180,6 +1258,14 @@ constexpr int MOE_GEMM_SLOTS_PER_EXPERT = 17;
 // refuses such batches.
 constexpr int MOE_PREFILL_SLOTS_PER_EXPERT = 32;
 
+// Grouped GEMM items hold up to 64 slots (32-row blocks by two, four
+// workgroups a CU) below this average of slots per expert, where few experts
+// pass 64; else 128 (two a CU), which decodes an expert's weights half as
+// often.  256 experts of 7168 x 2048 at 32 slots: gate + up 1218 against 1343
+// us, down 666 against 800; 16 experts of 4096 x 2048 at 64 / 128 / 1024
+// slots, a call: 180 against 156, 270 against 253, 1528 against 1373 us.
+constexpr int MOE_ITEM64_SLOTS = 48;
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace
@@ -1232,7 +1318,7 @@ MoeLayout moe_layout(const MoeArgs &a, bool generic_gu, bool generic_d) {
   // experts, and a repeated one would only be read twice)
   L.direct = !L.gemm && a.rows == 1 && a.inds != nullptr;
   const int item_rows = L.item_rows =
-      L.gemm ? RDG_ROWS : MOE_ITEM_ROWS;
+      !L.gemm ? MOE_ITEM_ROWS : slots < MOE_ITEM64_SLOTS * a.experts ? RDG_ROWS / 2 : RDG_ROWS;
   L.max_items = std::min(a.experts, slots) + (slots + item_rows - 1) / item_rows;
   const int groups = std::max(1, std::min(a.experts, slots));
   moe_plan(a.hidden, a.inter, 2 * groups, L.direct, &L.ks_gu, &L.tps_gu);
@@ -1403,9 +1489,11 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
     hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(MOE_ROUTE_THREADS), 0, s, a.inds, L.slots,
                        a.experts, sorted, items, n_items, (uint32_t)L.item_rows);
     uint16_t *xg = (uint16_t *)(base + L.xg), *xu = (uint16_t *)(base + L.xu);
-    const int nblk = a.hidden / 128;
-    hipLaunchKernelGGL(moe_prep_kernel, dim3((nblk + 3) / 4, L.slots), dim3(256), 0, s, a.x,
-                       a.xdt, a.inds, a.experts, a.topk, gate.suh, up.suh, xg, xu, a.hidden, nblk);
+    const uint32_t nblocks = (uint32_t)L.slots * (uint32_t)(a.hidden / 128);
+    const int wide = (((uintptr_t)a.x | (uintptr_t)gate.suh | (uintptr_t)up.suh) & 15) == 0;
+    hipLaunchKernelGGL(moe_prep_kernel, dim3((nblocks + 15) / 16), dim3(256), 0, s, a.x, a.xdt,
+                       a.inds, a.experts, a.topk, gate.suh, up.suh, xg, xu, a.hidden, nblocks,
+                       wide);
     auto grouped = [&](const MoeBank *const *b, const uint16_t *const *xp, uint16_t *const *yo,
                        int nw) {
       RdGroupArgs r{};
@@ -1425,18 +1513,16 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
       const unsigned grid = (unsigned)r.ct * ((L.max_items + 7) / 8 * 8);
       rate_dispatch(b[0]->f.n / 16, [&](auto KC) {
         constexpr int K = decltype(KC)::value;
-        if constexpr (K > 0) gemm_rd_grouped_go<K>(b[0]->f, grid, s, r);
+        if constexpr (K > 0) gemm_rd_grouped_go<K>(b[0]->f, L.item_rows, grid, s, r);
       });
     };
     const MoeBank *const gub[2] = {&gate, &up}, *const db[1] = {&down};
     const uint16_t *const gux[2] = {xg, xu}, *const dx[1] = {xd};
     uint16_t *const guy[2] = {g, u}, *const dy[1] = {d};
     grouped(gub, gux, guy, 2);
-    hipLaunchKernelGGL(moe_mid_kernel, dim3(a.inter / 128, L.slots), dim3(64), 0, s, g, u, a.inds,
-                       a.experts, down.suh, xd, a.inter, a.limit, -1, nullptr);
+    launch_moe_mid(g, u, a.inds, a.experts, down.suh, xd, L.slots, a.inter, a.limit, -1, nullptr, s);
     grouped(db, dx, dy, 1);
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((a.hidden + 255) / 256, a.rows), dim3(256), 0, s,
-                       d, a.inds, a.scores, a.sdt, a.topk, a.experts, a.hidden, a.y, a.ydt);
+    launch_moe_combine(a, d, s);
     return hipGetLastError();
   }
   const size_t gu_part = (size_t)L.ks_gu * L.slots * a.inter;
@@ -1494,9 +1580,8 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
   moe_gemv_launch(gate.f, grid_gu, gemv_lds_bytes(lds_rows, L.tps_gu, gu_generic), s, mgu,
                   isorted, iitems, in_items, a.topk);
   if (!fused_mid)
-    hipLaunchKernelGGL(moe_mid_kernel, dim3(a.inter / 128, L.slots), dim3(64), 0, s, g, u, a.inds,
-                       a.experts, down.suh, xd, a.inter, a.limit, sh_index,
-                       shared ? shared->down.suh : nullptr);
+    launch_moe_mid(g, u, a.inds, a.experts, down.suh, xd, L.slots, a.inter, a.limit, sh_index,
+                   shared ? shared->down.suh : nullptr, s);
   md.tw[0] = md.tw[1] = reinterpret_cast<const uint32_t *>(down.trellis);
   md.a.w[0] = moe_weight(down, d, pd);
   if (shared) {
@@ -1511,8 +1596,7 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
                        s, d, a.inds, a.scores, a.sdt, routes_k, a.experts, shared->logit,
                        shared->gate_vec, a.x, a.xdt, a.hidden, a.y, a.ydt);
   else
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((a.hidden + 255) / 256, a.rows), dim3(256), 0, s,
-                       d, a.inds, a.scores, a.sdt, a.topk, a.experts, a.hidden, a.y, a.ydt);
+    launch_moe_combine(a, d, s);
   return hipGetLastError();
 }
 
