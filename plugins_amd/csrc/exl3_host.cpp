@@ -956,9 +956,10 @@ static hipError_t run_linear(const exl3_weight *w, const WeightPriv *pv, const v
 // (row r g of the flattened [rows G, in] takes group g's suh), one grouped
 // GEMM launch over every group's 256-row tiles with the finish fused, y
 // written in place (turboexl3_ds41/src/woa_join.zig:1-5: one prepare and
-// one finish launch for all groups).  Otherwise per group: its rows gathered
-// into scratch by a strided 2-D copy, the linear's kernels (GEMV or GEMM by
-// the row count, as exl3_matmul), the result copied into y's group columns.
+// one finish launch for all groups).  Decode rows: one GEMV launch over every
+// group.  Otherwise (prompts at the half-integer rates) per group: its rows
+// gathered into scratch by a strided 2-D copy, the linear's GEMM, the result
+// copied into y's group columns.
 static exl3_verdict grouped_matmul(const exl3_weight *w, const WeightPriv *pv, exl3_array x,
                                    hipStream_t s, exl3_array *out) {
   const int xdt = act_of(x.dtype);
@@ -986,6 +987,26 @@ static exl3_verdict grouped_matmul(const exl3_weight *w, const WeightPriv *pv, e
       e = exl3::launch_gemm_groups((const uint16_t *)w->w.data, pv->f, (const uint16_t *)ss->xp,
                                    (const uint16_t *)w->biases.data, out->data, xdt, (int)rows,
                                    (int)G, (int)in, (int)outf, s);
+    return e == hipSuccess ? ok() : hip_failed(e);
+  }
+  // decode rows (and prompts at the rates without a GEMM, 16 rows at a time):
+  // every group in one GEMV launch, unless its offsets pass 32 bits
+  const bool generic = !pv->f.integer_rate();
+  const int wrows = (int)std::min<int64_t>(rows, exl3::GEMV_ROWS_MAX);
+  const int last = (int)((rows - 1) % exl3::GEMV_ROWS_MAX + 1);  // (may split k further)
+  const size_t pf = G > 65535 ? 0
+                              : std::max(exl3::gemv_groups_floats(wrows, (int)G, (int)in, (int)outf, generic),
+                                         exl3::gemv_groups_floats(last, (int)G, (int)in, (int)outf, generic));
+  if ((rows <= exl3::GEMV_ROWS_MAX || !pv->f.gemm_rate()) && G <= 65535 && pf * 4 < (1u << 31) &&
+      (int64_t)wrows * G * std::max(in, outf) < (int64_t)1 << 31) {
+    exl3::Scratch sc;
+    hipError_t e = slots_for(ss, pf, s, &sc);
+    for (int64_t r0 = 0; r0 < rows && e == hipSuccess; r0 += exl3::GEMV_ROWS_MAX)
+      e = exl3::launch_gemv_groups(
+          (const uint16_t *)w->w.data, pv->f, (const char *)x.data + (size_t)r0 * G * in * esz, xdt,
+          (const uint16_t *)w->scales.data, (const uint16_t *)w->biases.data,
+          (char *)out->data + (size_t)r0 * G * outf * esz, xdt,
+          (int)std::min<int64_t>(exl3::GEMV_ROWS_MAX, rows - r0), (int)G, (int)in, (int)outf, sc, s);
     return e == hipSuccess ? ok() : hip_failed(e);
   }
   const size_t xg_bytes = ((size_t)rows * in * esz + 255) & ~(size_t)255;

@@ -160,6 +160,9 @@ struct GemvCfg {
   int shared_expert;  // routed launches: the index of the shared expert (-1: none)
   int experts;        // routed launches without an item list: expert indices below this
   int routes_k;       // ... > 0: sorted holds k routes, slot k is the shared expert
+  // grouped linears (groups > 0, no item list): item z is linear z of the
+  // G-bank with the call's group_rows rows, whose slots are row * groups + z
+  int groups, group_rows;
   // attention prologue (set: on; the launch's x is then this pointer): the
   // decode attention's per-split slots [rows][attn_nkv][attn_nsplit]
   // [attn_g][128 + 2] (o values, then m, l)
@@ -1780,7 +1783,8 @@ static_assert(MOE_DIRECT_TPS_MAX / 8 <= PREP_GROUPS, "a one-row item's prepare e
 // sorted[z] (the routes; with a.c.routes_k = k > 0 slot k is the shared
 // expert), skipped when not below a.c.experts.  PRO_SWIGLU (down): x is
 // the slots' gate rows and a.c.x2 their up rows (topk 1: row slot), the
-// mid step's SwiGLU and rotation formed in the prepare.
+// mid step's SwiGLU and rotation formed in the prepare.  A grouped linear
+// (a.c.groups > 0) takes item z as its linear z over all the call's rows.
 template <int K, int CB, bool MASKED, int PRO>
 __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
     const uint32_t *tw0, const uint32_t *tw1, const void *x, uint32_t g0, uint32_t g1,
@@ -1792,6 +1796,8 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
   if (items != nullptr) {
     if ((uint32_t)item >= *n_items) return;
     it = items[item];
+  } else if (a.c.groups > 0) {
+    it = MoeItem{(uint32_t)item, 0u, (uint32_t)a.c.group_rows, 0u};
   } else {
     if ((size_t)item >= a.c.ptotal) return;
     // uniform across the workgroup; readfirstlane keeps it in a scalar
@@ -1809,7 +1815,9 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
   GemvRow *ri = reinterpret_cast<GemvRow *>(smem);
   if (threadIdx.x < GEMV_ROWS) {
     const int b = min((int)threadIdx.x, (int)it.count - 1);
-    const int slot = items != nullptr ? (int)sorted[it.start + b] : item;
+    const int slot = items != nullptr    ? (int)sorted[it.start + b]
+                     : a.c.groups > 0 ? b * a.c.groups + item
+                                      : item;
     const int in = geo.in_tiles * 16, out = out_tiles * 16;
     ri[threadIdx.x] = GemvRow{(geo.prepared ? slot : slot / topk) * in, slot * out, slot, 0};
   }
@@ -1829,7 +1837,9 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
     gemv_wg<K, CB, MASKED, decltype(P)::value, PRO>(twe, out_tiles, x, geo, a.c, Wx,
                                                sh ? 0 : (int)it.expert, (int)it.count, rm,
                                                blockIdx.x - ws.c0, blockIdx.y, smem + 256,
-                                               items != nullptr ? MOE_ITEM_ROWS : 1);
+                                               items != nullptr    ? MOE_ITEM_ROWS
+                                               : a.c.groups > 0 ? a.c.group_rows
+                                                                : 1);
   };
   const int items_n = (int)it.count * (geo.tps / 8);
   if (items_n <= PREP_ITEMS)

@@ -106,6 +106,13 @@ hipError_t launch_prepare(const void *x, int xdt, const uint16_t *suh, uint16_t 
 hipError_t launch_gemm_groups(const uint16_t *trellis, const Format &f, const uint16_t *xp,
                               const uint16_t *svh, void *y, int ydt, int rows, int groups,
                               int in, int out, hipStream_t s);
+// Up to GEMV_ROWS_MAX rows of a grouped linear in one GEMV launch (any rate):
+// x [rows, G, in] (ACT_*) -> y [rows, G, out] in ydt, both in place; sc holds
+// gemv_groups_floats partial sums.
+size_t gemv_groups_floats(int rows, int groups, int in, int out, bool generic);
+hipError_t launch_gemv_groups(const uint16_t *trellis, const Format &f, const void *x, int xdt,
+                              const uint16_t *suh, const uint16_t *svh, void *y, int ydt, int rows,
+                              int groups, int in, int out, const Scratch &sc, hipStream_t s);
 // finish: z f16 [rows, out] -> y [rows, out] (ACT_*); svh f16 [out].
 hipError_t launch_finish(const uint16_t *z, const uint16_t *svh, void *y, int ydt, int rows,
                          int out, hipStream_t s);

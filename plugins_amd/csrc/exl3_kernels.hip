@@ -1422,7 +1422,68 @@ MoeGemv moe_gemv(const void *x, int xdt, bool prepared, size_t slots, int in, in
   return m;
 }
 
+// The k-splits of a grouped linear's GEMV: the dense plan over every group's
+// column groups.
+void gemv_groups_plan(int rows, int groups, int in, int out, bool generic, int *ks, int *tps) {
+  gemv_plan(in, out, groups, rows, ks, tps, GEMV_TPS_MAX);
+  if (generic && *tps > 32) {
+    *tps = 32;
+    *ks = (in / 16 + 31) / 32;
+  }
+}
+
 }  // namespace
+
+size_t gemv_groups_floats(int rows, int groups, int in, int out, bool generic) {
+  int ks, tps;
+  gemv_groups_plan(rows, groups, in, out, generic, &ks, &tps);
+  return (size_t)ks * rows * groups * out;
+}
+
+// One launch of the grouped GEMV, group z its work item z: every group's
+// rows read and written in place.  (Per group, a strided copy in, a GEMV and a
+// copy out were 24 launches at 8 groups: 8 x 4096 -> 1024 at K = 3, 4 rows,
+// 104.7 -> 12.1 us.)
+hipError_t launch_gemv_groups(const uint16_t *trellis, const Format &f, const void *x, int xdt,
+                              const uint16_t *suh, const uint16_t *svh, void *y, int ydt, int rows,
+                              int groups, int in, int out, const Scratch &sc, hipStream_t s) {
+  if (rows < 1 || rows > GEMV_ROWS_MAX || groups < 1 || groups > 65535 || in <= 0 || out <= 0 ||
+      in % 128 != 0 || out % 128 != 0 || in / 16 > 65535 || out / 128 > 65535 || y == nullptr)
+    return hipErrorInvalidValue;
+  if (f.n < 16 || f.n > 128 || (f.n & 1)) return hipErrorInvalidValue;
+  if ((int64_t)rows * groups * std::max(in, out) >= (int64_t)1 << 31) return hipErrorInvalidValue;
+  const bool generic = !f.integer_rate();
+  int ks, tps;
+  gemv_groups_plan(rows, groups, in, out, generic, &ks, &tps);
+  const size_t slots = (size_t)rows * groups;
+  // a split's slot planes are addressed with 32-bit byte offsets
+  if (ks > GEMV_KSPLIT_MAX || (size_t)ks * slots * out * 4 > 0x7FFFFFFFu)
+    return hipErrorInvalidValue;
+  if (rows * (tps / 8) > PREP_PASSES * PREP_GROUPS) return hipErrorInvalidValue;
+  if (ks > 1 && (sc.partial == nullptr || sc.status == nullptr ||
+                 sc.partial_floats < (size_t)ks * slots * out))
+    return hipErrorInvalidValue;
+  MoeGemv m = moe_gemv(x, xdt, false, slots, in, out, f, ks, tps);
+  m.nweights = 1;
+  m.a.c.ydt = ydt;
+  m.a.c.status = sc.status;
+  m.a.c.poll_max = splitk_poll_max();
+  m.a.c.drop_partials = splitk_drop();
+  m.a.c.groups = groups;
+  m.a.c.group_rows = rows;
+  m.tw[0] = m.tw[1] = reinterpret_cast<const uint32_t *>(trellis);
+  GemvWeight &w = m.a.w[0];
+  w.suh = suh;
+  w.svh = svh;
+  w.y = y;
+  w.partial = sc.partial;
+  w.expert_words = (size_t)(in / 16) * (out / 16) * (f.n / 2);
+  const dim3 grid(out / 128, ks, groups);
+  uint32_t g[3];
+  if (!moe_geo(m, grid, &g[0], &g[1], &g[2])) return hipErrorInvalidValue;
+  moe_gemv_launch(f, grid, gemv_lds_bytes(rows, tps, generic), s, m, nullptr, nullptr, nullptr, 1);
+  return hipGetLastError();
+}
 
 bool moe_shared_direct(const MoeArgs &a, bool gu_generic, bool d_generic) {
   if (a.rows != 1 || a.topk <= 0 || a.experts <= 0 || a.hidden % 128 != 0) return false;
