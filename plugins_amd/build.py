@@ -36,7 +36,8 @@ HOST_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-par
 # in parallel.
 SOURCES = [
     ("exl3_kernels.hip", "exl3_kernels", DEVICE_FLAGS),
-    *[("exl3_rate.hip", f"exl3_rate_k{k}", DEVICE_FLAGS + [f"-DEXL3_INST_K={k}"]) for k in range(9)],
+    *[("exl3_rate.hip", f"exl3_rate_k{k}", DEVICE_FLAGS + [f"-DEXL3_INST_K={k}"])
+      for k in [*range(9), -3, -5]],
     *[("exl3_rate_gemm.hip", f"exl3_rate_gemm_k{k}", DEVICE_FLAGS + [f"-DEXL3_INST_K={k}"])
       for k in range(9)],
     ("decoder_ops.hip", "decoder_ops", DEVICE_FLAGS),

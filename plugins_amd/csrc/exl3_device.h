@@ -301,6 +301,34 @@ __device__ __forceinline__ uint32_t chunk_pair_mul1_h(const uint32_t (&w)[K + 1]
 constexpr float MUL1_A = 0.00676727294921875f;
 constexpr float MUL1_B = -10.3828125f;
 
+// ------------------------------------------------ half-integer rates
+//
+// At n = 8 FR halfwords a tile (FR odd: K = FR / 2 = 1.5, 2.5, exllamav3's
+// half-integer rates; turboexl3_ds41/src/bank/frac.zig:1-21), chunk c of a
+// tile (codewords 32 c .. 32 c + 31) is stream halfwords c FR .. c FR + FR - 1
+// (bitEnd(32 c) = 2 n c: a halfword boundary, not a dword one).  A decode
+// thread loads the LW = NB + 1 dwords holding that chunk and the halfword
+// before it (the tile's last for c = 0: the ring wraps), starting at dword b;
+// one v_alignbit_b32 per dword by sh (16 when that history halfword is the
+// low half of dword b, else 0 with b one dword earlier) leaves NB dwords
+// [history | chunk], MSB first, in which codeword i's window ends at bit
+// 16 + floor((i + 1) FR / 2): compile-time positions, as chunk_cw's.
+template <int FR>
+constexpr int gf_nb() {
+  return (FR + 1) / 2;
+}
+
+template <int FR, int I>
+__device__ __forceinline__ uint32_t chunk_cw_frac(const uint32_t (&w)[gf_nb<FR>()]) {
+  constexpr int E = 16 + ((I + 1) * FR) / 2;
+  constexpr int J0 = (E - 16) >> 5, J1 = (E - 1) >> 5;
+  static_assert(J1 < gf_nb<FR>(), "window outside the chunk buffer");
+  if constexpr (J0 == J1)
+    return __builtin_amdgcn_ubfe(w[J0], 31 - ((E - 1) & 31), 16);
+  else
+    return __builtin_amdgcn_alignbit(w[J0], w[J1], 31 - ((E - 1) & 31)) & 0xFFFFu;
+}
+
 // ------------------------------------------------------------ generic rate
 
 // Codeword t (0..255) of a tile of n halfwords whose n/2 dwords are in `tw`

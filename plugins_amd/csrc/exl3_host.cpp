@@ -922,7 +922,7 @@ static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *co
   for (int64_t r0 = 0; r0 < rows; r0 += exl3::GEMV_ROWS_MAX) {
     const int r = (int)std::min<int64_t>(exl3::GEMV_ROWS_MAX, rows - r0);
     exl3::Scratch sc[4];
-    hipError_t e = gemv_scratch(ss, outs, count, in, r, !p0->f.integer_rate(), sc, s);
+    hipError_t e = gemv_scratch(ss, outs, count, in, r, p0->f.gemv_generic(), sc, s);
     if (e != hipSuccess) return e;
     exl3::GemvLinear ls[4];
     for (int i = 0; i < count; ++i) {
@@ -991,7 +991,7 @@ static exl3_verdict grouped_matmul(const exl3_weight *w, const WeightPriv *pv, e
   }
   // decode rows (and prompts at the rates without a GEMM, 16 rows at a time):
   // every group in one GEMV launch, unless its offsets pass 32 bits
-  const bool generic = !pv->f.integer_rate();
+  const bool generic = pv->f.gemv_generic();
   const int wrows = (int)std::min<int64_t>(rows, exl3::GEMV_ROWS_MAX);
   const int last = (int)((rows - 1) % exl3::GEMV_ROWS_MAX + 1);  // (may split k further)
   const size_t pf = G > 65535 ? 0
@@ -1097,7 +1097,7 @@ exl3_verdict exl3_matmul_noalloc(const exl3_weight *w, exl3_array x, exl3_stream
     const int outs[1] = {(int)pv->out};
     slot_floats = gemv_slot_need(outs, 1, (int)pv->in,
                                  (int)std::min<int64_t>(rows, exl3::GEMV_ROWS_MAX),
-                                 !pv->f.integer_rate());
+                                 pv->f.gemv_generic());
   }
   if (exl3::SLOT_HEADER_BYTES + slot_floats * 4 > exl3::NOALLOC_SLOT_BYTES ||
       xp_bytes + kpart_bytes > exl3::NOALLOC_BYTES - exl3::NOALLOC_SLOT_BYTES)
@@ -1248,7 +1248,7 @@ exl3_verdict exl3_swiglu(const exl3_weight *gate, const exl3_weight *up, const e
     if (e != hipSuccess) return hip_failed(e);
     const int outs[1] = {(int)hidden};
     exl3::Scratch sc;
-    e = gemv_scratch(ss, outs, 1, (int)pd->in, (int)rows, !pd->f.integer_rate(), &sc, s);
+    e = gemv_scratch(ss, outs, 1, (int)pd->in, (int)rows, pd->f.gemv_generic(), &sc, s);
     if (e != hipSuccess) return hip_failed(e);
     const exl3::GemvLinear l{(const uint16_t *)down->w.data, (const uint16_t *)down->scales.data,
                              (const uint16_t *)down->biases.data, out->data, nullptr, (int)hidden};
@@ -2086,7 +2086,7 @@ int exl3d_linears(const exl3_weight *const *ws, int count, const void *x, int B,
     ls[i].out = wouts[i];
   }
   exl3::Scratch sc[4];
-  hipError_t e = gemv_scratch(ss, wouts, count, in, B, !pvs[0]->f.integer_rate(), sc, s);
+  hipError_t e = gemv_scratch(ss, wouts, count, in, B, pvs[0]->f.gemv_generic(), sc, s);
   if (e != hipSuccess) return e;
   exl3::GemvFuse fz;
   fz.up = up;
@@ -2098,7 +2098,7 @@ int exl3d_linears(const exl3_weight *const *ws, int count, const void *x, int B,
   int xdt = norm_w ? exl3::ACT_F32 : exl3::ACT_F16;
   int total = 0;
   for (int i = 0; i < count; ++i) total += wouts[i];
-  const bool pre_norm = norm_w && (!exl3::gemv_one_batch(in, total, !pvs[0]->f.integer_rate(), B) ||
+  const bool pre_norm = norm_w && (!exl3::gemv_one_batch(in, total, pvs[0]->f.gemv_generic(), B) ||
                                    in / 128 > exl3::NORM_MAXBLK);
   const bool pre_swiglu = up && B > exl3::SWIGLU_PROLOGUE_ROWS;
   // rows the prologue does not take: the RMSNorm (of h as it stands) or the
@@ -2159,7 +2159,7 @@ int exl3d_attn_o(const uint16_t *q, const uint16_t *k, const uint16_t *v, const 
   const int G = exl3d_attn_heads_per_kv();
   const int ns = exl3d_attn_splits(B, nkv, Tmax);
   if (ns < 1 || nq != G * nkv || pv->in != (int64_t)nq * EXL3D_HEAD_DIM) return -1;
-  const bool fused = exl3::gemv_one_batch((int)pv->in, (int)pv->out, !pv->f.integer_rate(), B);
+  const bool fused = exl3::gemv_one_batch((int)pv->in, (int)pv->out, pv->f.gemv_generic(), B);
   if (!fused && !att) return -1;
   if (hipSetDevice(pv->device) != hipSuccess) return hipErrorInvalidDevice;
   int r = exl3d_attn_decode_rope(q, k, v, qn, kn, pos, B, nq, nkv, eps, theta, kcache, vcache,
@@ -2183,7 +2183,7 @@ int exl3d_attn_o(const uint16_t *q, const uint16_t *k, const uint16_t *v, const 
     l.zout = nullptr;
     l.out = wout;
     exl3::Scratch sc;
-    e = gemv_scratch(ss, &wout, 1, in, B, !pv->f.integer_rate(), &sc, s);
+    e = gemv_scratch(ss, &wout, 1, in, B, pv->f.gemv_generic(), &sc, s);
     if (e != hipSuccess) return e;
     exl3::GemvFuse fz;
     fz.res = res;
@@ -2205,7 +2205,7 @@ int exl3d_attn_o(const uint16_t *q, const uint16_t *k, const uint16_t *v, const 
   l.zout = nullptr;
   l.out = wout;
   exl3::Scratch sc;
-  hipError_t e = gemv_scratch(ss, &wout, 1, in, B, !pv->f.integer_rate(), &sc, s);
+  hipError_t e = gemv_scratch(ss, &wout, 1, in, B, pv->f.gemv_generic(), &sc, s);
   if (e != hipSuccess) return e;
   exl3::GemvFuse fz;
   fz.res = res;

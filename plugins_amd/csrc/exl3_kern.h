@@ -942,13 +942,17 @@ __device__ __forceinline__ void gemv_wg(const uint32_t *twe, int out_tiles, cons
   uint16_t *xs = reinterpret_cast<uint16_t *>(smem);
   const int zrows = rows_alloc > 2 ? rows_alloc : 2;
   float *zp = reinterpret_cast<float *>(smem + (size_t)rows_alloc * kr * 2);  // [2][zrows][128]
-  // mul1 at an integer rate: the MFMAs take h (the codebook value before its
-  // affine step, chunk_pair_mul1_h), and z = a * acc + b * (sum of the
-  // k-part's prepared activations) afterwards, from the 64-element sums
-  // hsum[row][ntk / 4] that the prepare leaves
+  // K: 1..8 an integer rate; -FR the half-integer rate n = 8 FR; 0 any even n
+  // with run-time windows.  mul1 at an integer rate: the MFMAs take h (the
+  // codebook value before its affine step, chunk_pair_mul1_h), and z = a * acc
+  // + b * (sum of the k-part's prepared activations) afterwards, from the
+  // 64-element sums hsum[row][ntk / 4] that the prepare leaves.  (This skips
+  // the codebook's rounding of each weight to f16, 2e-4 of the result; the
+  // half-integer rates keep it.)
+  constexpr int FR = K < 0 ? -K : 1;
   constexpr bool FOLD = K > 0 && CB == CB_MUL1;
   float *hsum = zp + 2 * zrows * 128;
-  const int nw = K > 0 ? 8 * K : a.nw;  // trellis dwords per tile
+  const int nw = K > 0 ? 8 * K : K < 0 ? 4 * FR : a.nw;  // trellis dwords per tile
   const int g = lane >> 4, t = (lane >> 3) & 1, c = lane & 7;
   const size_t tn = (size_t)cg * 8 + 2 * q + t;
   const int part = ntk >> 1;  // k-tile rows per k-part, a multiple of 4
@@ -961,11 +965,31 @@ __device__ __forceinline__ void gemv_wg(const uint32_t *twe, int out_tiles, cons
   // the next NBUF - 1 steps' weights (steps past the last reload the last one:
   // in bounds and unused, so no branches and the waits stay exact), svh for
   // the finish.
-  constexpr int KB = K > 0 ? K : 1;
+  constexpr int KB = K > 0 ? K : K < 0 ? gf_nb<FR>() + 1 : 1;
   // steps in flight per wave: as many as a few registers allow
-  constexpr int NBUF = K <= 0 ? 1 : 3;
+  constexpr int NBUF = K == 0 ? 1 : 3;
   uint32_t bw[NBUF][KB];
-  const gu32_t *wp = (const gu32_t *)(twe + ((size_t)(kb + g) * out_tiles + tn) * nw + c * K);
+  // half-integer rates: the lane's chunk and the halfword before it are KB
+  // dwords of its tile from dword hs / 2 - (0 or 1) on (hs the history
+  // halfword, gw_decode_frac's layout); all but the first are consecutive, the
+  // first wraps for chunk 0
+  const int hs = (c * FR - 1 + 8 * FR) % (8 * FR);
+  const bool hlow = (hs & 1) != 0;
+  const int b1 = ((hs >> 1) + (hlow ? 1 : 0)) % (4 * FR);  // the second dword
+  const int d0 = b1 == 0 ? 4 * FR - 1 : -1;                // the first, from it
+  const uint32_t fsh = hlow ? 16u : 0u;
+  const gu32_t *wp = (const gu32_t *)(twe + ((size_t)(kb + g) * out_tiles + tn) * nw +
+                                      (K < 0 ? b1 : c * K));
+  auto load_words = [&](uint32_t(&b)[KB], const gu32_t *p) {
+    if constexpr (K < 0) {
+      b[0] = p[d0];
+#pragma unroll
+      for (int i = 1; i < KB; ++i) b[i] = p[i - 1];
+    } else {
+#pragma unroll
+      for (int i = 0; i < KB; ++i) b[i] = p[i];
+    }
+  };
   const size_t wstep = (size_t)4 * out_tiles * nw;  // dwords per step
   const int nb = ntk >> 3, nitems = nrows * nb;
   // ONEB: one item (row, 128-block) per wave and batch; else every row's
@@ -989,10 +1013,7 @@ __device__ __forceinline__ void gemv_wg(const uint32_t *twe, int out_tiles, cons
     else
       gemv_rows_load_su(x, geo.prepared, psuh + (size_t)expert * in, nitems, nb, tk0, rr);
   }
-  if constexpr (K > 0) {
-#pragma unroll
-    for (int i = 0; i < K; ++i) bw[0][i] = wp[i];
-  }
+  if constexpr (K != 0) load_words(bw[0], wp);
   // attention prologue: the first round of the wave's first item (x is the
   // attention's split slots)
   AttnLoads al;
@@ -1029,13 +1050,9 @@ __device__ __forceinline__ void gemv_wg(const uint32_t *twe, int out_tiles, cons
     static_assert(ONEB, "the RMSNorm prologue is for rows that fit one prepare batch");
     gemv_prep_load_norm(a, rm, nitems, nb, tk0, in, 0, wave, lane, pr);
   }
-  if constexpr (K > 0) {
+  if constexpr (K != 0) {
 #pragma unroll
-    for (int b = 1; b < NBUF; ++b) {
-      const gu32_t *pb = wp + (size_t)min(b, iters - 1) * wstep;
-#pragma unroll
-      for (int i = 0; i < K; ++i) bw[b][i] = pb[i];
-    }
+    for (int b = 1; b < NBUF; ++b) load_words(bw[b], wp + (size_t)min(b, iters - 1) * wstep);
   }
   // svh of this lane's two columns (read whether or not the finish runs: a
   // load without a branch around it)
@@ -1072,20 +1089,21 @@ __device__ __forceinline__ void gemv_wg(const uint32_t *twe, int out_tiles, cons
   const int arow = min(lane & 15, nrows - 1);
   const uint16_t *xa = xs + arow * kr + (kp * part + g) * 16;
   f4_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
-  if constexpr (K > 0) {
+  if constexpr (K != 0) {
     const int src = ((lane & ~7) | ((lane + 7) & 7)) << 2;
     auto step = [&](uint32_t(&b)[KB], int it) {
-      uint32_t wd[K + 1];
+      uint32_t wd[K > 0 ? K + 1 : gf_nb<FR>()];
+      if constexpr (K > 0) {
 #pragma unroll
-      for (int i = 0; i < K; ++i) wd[i + 1] = b[i];
-      wd[0] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)b[K - 1]);
-      {
-        // the buffer is free once copied: its next step's load goes out
-        // before this step's decode
-        const gu32_t *pn = wp + (size_t)min(it + NBUF, iters - 1) * wstep;
+        for (int i = 0; i < K; ++i) wd[i + 1] = b[i];
+        wd[0] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)b[K - 1]);
+      } else {
 #pragma unroll
-        for (int i = 0; i < K; ++i) b[i] = pn[i];
+        for (int i = 0; i < KB - 1; ++i) wd[i] = __builtin_amdgcn_alignbit(b[i], b[i + 1], fsh);
       }
+      // the buffer is free once copied: its next step's load goes out before
+      // this step's decode
+      load_words(b, wp + (size_t)min(it + NBUF, iters - 1) * wstep);
       const h8_t alo = *reinterpret_cast<const h8_t *>(xa + it * 64);
       const h8_t ahi = *reinterpret_cast<const h8_t *>(xa + it * 64 + 8);
       // one B operand at a time (pairs f, f+4, f+8, f+12: rows 0-7 or 8-15 of
@@ -1096,7 +1114,10 @@ __device__ __forceinline__ void gemv_wg(const uint32_t *twe, int out_tiles, cons
         uint32_t qv[4];
         static_for<4>([&](auto J) {
           constexpr int pq = p0 + 4 * decltype(J)::value;
-          if constexpr (FOLD)
+          if constexpr (K < 0)
+            qv[J] = decode_pair_cw<CB, MASKED>(chunk_cw_frac<FR, 2 * pq>(wd),
+                                               chunk_cw_frac<FR, 2 * pq + 1>(wd), a.dec);
+          else if constexpr (FOLD)
             qv[J] = chunk_pair_mul1_h<MASKED, K, pq>(wd, a.dec.mask);
           else
             qv[J] = chunk_pair_cw<K, CB, MASKED, pq>(wd, a.dec);
@@ -1564,34 +1585,6 @@ __device__ __forceinline__ void gw_decode_main(uint16_t *lds, const uint32_t *tw
   }
 }
 
-// ------------------------------------------------ half-integer rates
-//
-// At n = 8 FR halfwords a tile (FR odd: K = FR / 2 = 1.5, 2.5, exllamav3's
-// half-integer rates; turboexl3_ds41/src/bank/frac.zig:1-21), chunk c of a
-// tile (codewords 32 c .. 32 c + 31) is stream halfwords c FR .. c FR + FR - 1
-// (bitEnd(32 c) = 2 n c: a halfword boundary, not a dword one).  A decode
-// thread loads the LW = NB + 1 dwords holding that chunk and the halfword
-// before it (the tile's last for c = 0: the ring wraps), starting at dword b;
-// one v_alignbit_b32 per dword by sh (16 when that history halfword is the
-// low half of dword b, else 0 with b one dword earlier) leaves NB dwords
-// [history | chunk], MSB first, in which codeword i's window ends at bit
-// 16 + floor((i + 1) FR / 2): compile-time positions, as chunk_cw's.
-template <int FR>
-constexpr int gf_nb() {
-  return (FR + 1) / 2;
-}
-
-template <int FR, int I>
-__device__ __forceinline__ uint32_t chunk_cw_frac(const uint32_t (&w)[gf_nb<FR>()]) {
-  constexpr int E = 16 + ((I + 1) * FR) / 2;
-  constexpr int J0 = (E - 16) >> 5, J1 = (E - 1) >> 5;
-  static_assert(J1 < gf_nb<FR>(), "window outside the chunk buffer");
-  if constexpr (J0 == J1)
-    return __builtin_amdgcn_ubfe(w[J0], 31 - ((E - 1) & 31), 16);
-  else
-    return __builtin_amdgcn_alignbit(w[J0], w[J1], 31 - ((E - 1) & 31)) & 0xFFFFu;
-}
-
 // The decode waves' main loop at a half-integer rate: gw_decode_main's
 // schedule and barriers (stage st + 1 decoded during stage st into B buffer
 // (st + 1) % 2) with each thread's chunk loaded whole (off: its LW dword
@@ -1960,7 +1953,7 @@ inline void cb_dispatch(const Format &f, G &&go) {
              : go(std::integral_constant<int, CB_HASH>{}, F{});
       break;
     case CB_PAIR1:
-      if constexpr (K == 0 || (K >= 2 && K <= 4)) go(std::integral_constant<int, CB_PAIR1>{}, F{});
+      if constexpr (K <= 0 || (K >= 2 && K <= 4)) go(std::integral_constant<int, CB_PAIR1>{}, F{});
       break;
     default:
       masked ? go(std::integral_constant<int, CB_MUL1>{}, T{})
@@ -1985,7 +1978,8 @@ void gemm_grouped_go(const Format &f, dim3 grid, hipStream_t s, const uint32_t *
 
 // ====================================================== per-rate launchers
 //
-// K = 1..8: an integer rate (n = 16K) with compile-time windows; K = 0: any
+// K = 1..8: an integer rate (n = 16K) with compile-time windows; K = -3, -5:
+// the half-integer rates n = 8 |K|, likewise (GEMV only); K = 0: any
 // even n (GEMV only).
 
 // Dense GEMV over up to four weights (tw[i] their trellis words).
@@ -2131,6 +2125,8 @@ void gemm_frac_go(const Format &f, dim3 grid, hipStream_t s, const uint32_t *tw,
 #define EXL3_EXTERN_RATE(KK)            \
   extern template EXL3_GEMV_GO(KK);     \
   extern template EXL3_MOE_GEMV_GO(KK);
+EXL3_EXTERN_RATE(-5)
+EXL3_EXTERN_RATE(-3)
 EXL3_EXTERN_RATE(0)
 EXL3_EXTERN_RATE(1)
 EXL3_EXTERN_RATE(2)

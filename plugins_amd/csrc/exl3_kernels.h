@@ -40,6 +40,8 @@ struct Format {
   // the prefill GEMM's rates: the integer ones and the half-integer n = 24, 40
   // (exllamav3's K 1.5 and 2.5; turboexl3_ds41/src/bank/frac.zig:42-44)
   bool gemm_rate() const { return integer_rate() || n == 24 || n == 40; }
+  // the GEMV's run-time window form (its word stage in LDS, shorter splits)
+  bool gemv_generic() const { return !gemm_rate(); }
   CbRow dec() const {
     CbRow d;
     d.mask = mask();

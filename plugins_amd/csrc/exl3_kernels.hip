@@ -464,7 +464,15 @@ void gemv_multi_plan(int in, int total_out, bool generic, int rows, int *ksplit,
   }
 }
 
-// Calls launch(integral_constant<int, K>) for K = kk in 1..8, K = 0 otherwise.
+// The GEMV kernels' rate of a format (their K): 1..8, -3 and -5 (n = 24, 40)
+// or 0.  A half-integer rate's windows are as fixed as an integer rate's; with
+// run-time windows out of LDS its GEMV ran 24.0 us on q + k + v of 4096 at n =
+// 40, 3 rows, against 11.4.
+static int gemv_rate(const Format &f) {
+  return f.integer_rate() ? f.n / 16 : f.n == 24 ? -3 : f.n == 40 ? -5 : 0;
+}
+
+// Calls launch(integral_constant<int, K>) for K = kk in 1..8, -3, -5, else 0.
 template <typename F>
 static void rate_dispatch(int kk, F &&launch) {
   switch (kk) {
@@ -476,6 +484,8 @@ static void rate_dispatch(int kk, F &&launch) {
     case 6: launch(std::integral_constant<int, 6>{}); break;
     case 7: launch(std::integral_constant<int, 7>{}); break;
     case 8: launch(std::integral_constant<int, 8>{}); break;
+    case -3: launch(std::integral_constant<int, -3>{}); break;
+    case -5: launch(std::integral_constant<int, -5>{}); break;
     default: launch(std::integral_constant<int, 0>{});
   }
 }
@@ -486,7 +496,7 @@ static hipError_t gemv_multi(const GemvLinear *ls, int count, const Format &f, c
   if (count < 1 || count > GEMV_MAXW || rows < 1 || rows > GEMV_ROWS_MAX) return hipErrorInvalidValue;
   if (in <= 0 || in % 128 != 0) return hipErrorInvalidValue;
   if (f.n < 16 || f.n > 128 || (f.n & 1)) return hipErrorInvalidValue;
-  const bool generic = !f.integer_rate();
+  const bool generic = f.gemv_generic();
   int maxout = 0, totcg = 0;
   for (int i = 0; i < count; ++i) {
     if (ls[i].out <= 0 || ls[i].out % 128 != 0) return hipErrorInvalidValue;
@@ -578,7 +588,7 @@ static hipError_t gemv_multi(const GemvLinear *ls, int count, const Format &f, c
        fz.up != nullptr || fz.attn_nkv < 1 || fz.attn_g < 1 || fz.attn_nsplit < 1 ||
        in != fz.attn_nkv * fz.attn_g * 128))
     return hipErrorInvalidValue;
-  rate_dispatch(generic ? 0 : f.n / 16, [&](auto KC) {
+  rate_dispatch(gemv_rate(f), [&](auto KC) {
     gemv_go<decltype(KC)::value>(f, prep, grid, lds, s, tw, x, g0, g1, g2, a);
   });
   return hipGetLastError();
@@ -1386,7 +1396,7 @@ void moe_gemv_launch(const Format &f, dim3 grid, size_t lds, hipStream_t s, cons
                      int topk) {
   uint32_t g0, g1, g2;
   if (!moe_geo(m, grid, &g0, &g1, &g2)) return;  // checked before the first launch
-  rate_dispatch(f.integer_rate() ? f.n / 16 : 0, [&](auto KC) {
+  rate_dispatch(gemv_rate(f), [&](auto KC) {
     moe_gemv_go<decltype(KC)::value>(f, m.pro, grid, lds, s, m.tw[0], m.tw[1], m.x, g0, g1, g2,
                                      topk, sorted, items, n_items, m.a);
   });
@@ -1452,7 +1462,7 @@ hipError_t launch_gemv_groups(const uint16_t *trellis, const Format &f, const vo
     return hipErrorInvalidValue;
   if (f.n < 16 || f.n > 128 || (f.n & 1)) return hipErrorInvalidValue;
   if ((int64_t)rows * groups * std::max(in, out) >= (int64_t)1 << 31) return hipErrorInvalidValue;
-  const bool generic = !f.integer_rate();
+  const bool generic = f.gemv_generic();
   int ks, tps;
   gemv_groups_plan(rows, groups, in, out, generic, &ks, &tps);
   const size_t slots = (size_t)rows * groups;

@@ -1,7 +1,8 @@
 // exl3_rate.hip -- one rate's instantiation of the EXL3 GEMV and grouped MoE
-// GEMV kernels.  The build compiles this file once per K (0..8) with
-// -DEXL3_INST_K=K: K = 1..8 are the integer rates n = 16K with compile-time
-// bit windows, K = 0 the run-time window form for any even n.
+// GEMV kernels.  The build compiles this file once per K with -DEXL3_INST_K=K:
+// K = 1..8 are the integer rates n = 16K with compile-time bit windows, K = -3
+// and -5 the half-integer rates n = 24 and 40, K = 0 the run-time window form
+// for any even n.
 #include "exl3_kern.h"
 
 #ifndef EXL3_INST_K
