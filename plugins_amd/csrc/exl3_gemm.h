@@ -28,6 +28,11 @@ namespace exl3 {
 // two VALU slots, so the decode outweighs the MFMAs below 128 rows and is
 // half of them at 256.
 constexpr int RD_BK = 64;
+// The dense GEMM's workgroup shapes (gemm_rd_plan chooses).
+struct RdShape {
+  int mr, cw, kp;
+};
+constexpr RdShape RD_SHAPES[] = {{1, 4, 2}, {2, 4, 2}, {4, 4, 2}};
 __host__ __device__ constexpr int rd_threads(int CW, int KP) { return 64 * CW * KP; }
 // finish exchange: 32 rows of the 64 CW columns (f32), rows padded so that a
 // 16-row run of 16-byte stores touches distinct banks; rd_pass of them (with
@@ -427,8 +432,7 @@ __device__ __forceinline__ void rd_store(const float *fx, int tid, int rows, R &
 // The end of a tile: the k-parts' sums added (part 0 + part 1), then either
 // into a split's plane or finished.  With two k-parts row blocks go in pairs,
 // each part's waves owning one block of the pair.  rows: valid rows of the tile;
-// plane: f32 [row block][CW column waves][8][64 lanes][4] of this split and
-// tile (null: finish).
+// plane: f32 [rows][out] of this split at the tile's first row (null: finish).
 template <int MR, int CW, int KP, typename R>
 __device__ __forceinline__ void rd_end(f16v_t (&acc)[MR][2], char *smem, int rows, R &&orow,
                                        size_t out, int col0, int ncols, float *plane,
@@ -446,10 +450,12 @@ __device__ __forceinline__ void rd_end(f16v_t (&acc)[MR][2], char *smem, int row
   // a finished-sum block of the wave into its plane, or rotated into fx
   auto emit = [&](f16v_t (&v)[2], int ib, int region) {
     if (plane != nullptr) {
-      if (32 * ib < rows) {
-        float *p = plane + (size_t)ib * (2048 * CW) + cw * 2048 + lane * 4;
+      // (32-byte runs a row: a lane holds four consecutive columns)
+      if (32 * ib + (lane & 31) < rows && 64 * cw < ncols) {
+        float *p = plane + (size_t)(32 * ib + (lane & 31)) * out + col0 + 64 * cw + 4 * h;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) *reinterpret_cast<f4_t *>(p + q * 256) = quad(v, q);
+        for (int q = 0; q < 8; ++q)
+          *reinterpret_cast<f4_t *>(p + 16 * (q & 3) + 8 * (q >> 2)) = quad(v, q);
       }
     } else {
       if (y != nullptr) rd_rotate64(v, h);
@@ -505,6 +511,90 @@ __device__ __forceinline__ void rd_end(f16v_t (&acc)[MR][2], char *smem, int row
           out, col0, ncols, svh, y, ydt, zout);
     lds_barrier();
   });
+}
+
+// The dense GEMM over up to four linears that share rows, rate and codebook
+// (each with its own prepared rows), column tiles side by side in grid x, row
+// tiles in y, k-splits in z.
+constexpr int RD_MAXW = 4;
+struct RdWeight {
+  const uint32_t *tw;
+  const uint16_t *xp;   // [M][in]
+  const uint16_t *svh;
+  void *y;              // finished output in ydt, or null: zout
+  uint16_t *zout;       // f16(z)
+  float *kpart;         // split k: planes [split][M][out]
+  int out_tiles;
+  int ct0;              // first column tile in the grid
+};
+struct RdArgs {
+  RdWeight w[RD_MAXW];
+  int nw, ydt, M, in_tiles;
+  CbRow dec;
+};
+
+template <int K, int CB, bool MASKED, int MR, int CW, int KP, int FR>
+__global__ __launch_bounds__(rd_threads(CW, KP), (rd_waves<K, FR, MR, CW, KP>())) void
+gemm_rd_kernel(RdArgs a) {
+  __shared__ __attribute__((aligned(16))) char smem[rd_lds_bytes<K, FR, MR, CW, KP>()];
+  constexpr int COLS = 64 * CW, CT = 4 * CW;  // columns and tiles of a column tile
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cw = wave % CW, kp = wave / CW;
+  // Workgroup n runs on XCD n % 8 (the dispatcher's round robin); taking the
+  // row tile as n % (row tiles) gives each XCD a few row tiles of the
+  // activations to keep in its L2.  (Only the speed depends on this.)
+  const int mtiles = gridDim.y;
+  const int lin = blockIdx.x + gridDim.x * blockIdx.y;
+  const int gx = lin / mtiles, mt = lin % mtiles;
+  const int m0 = mt * (32 * MR);
+  int wi = 0;
+#pragma unroll
+  for (int i = 1; i < RD_MAXW; ++i)
+    if (i < a.nw && gx >= a.w[i].ct0) wi = i;
+  const RdWeight &W = a.w[wi];
+  const int ct = gx - W.ct0;
+  const int M = a.M, in = a.in_tiles * 16;
+  const int out_tiles = W.out_tiles;
+  const int ncols = min(COLS, out_tiles * 16 - ct * COLS);
+  // k range: whole 128-input blocks per split; with two k-parts the first
+  // half of the split's stages to part 0, the rest to part 1
+  const int S = gridDim.z, ks = blockIdx.z;
+  const int P = a.in_tiles / 8;
+  const int p0 = (int)((long)P * ks / S), p1 = (int)((long)P * (ks + 1) / S);
+  const int stages = (p1 - p0) * 2 / KP;    // of each k-part
+  const int st0 = 2 * p0 + kp * stages;     // the part's first stage
+
+  constexpr int NA = 4 * MR / CW;
+  uint32_t va[NA];
+#pragma unroll
+  for (int u = 0; u < NA; ++u) {
+    const int R = 8 * (NA * cw + u) + (lane >> 3);
+    const int q = (lane & 7) ^ ((R >> 1) & 7);
+    va[u] = (uint32_t)(((size_t)min(m0 + R, M - 1) * in + 8 * q) * 2);
+  }
+  constexpr int NW = rd_nw<K, FR>();
+  RdSrc src;
+  src.x = (const char *)W.xp + (size_t)st0 * (RD_BK * 2);
+  src.wrow = (uint32_t)out_tiles * (NW * 4);
+  // (columns past the last: the tile's first half again, not stored)
+  const int cwe = 64 * cw < ncols ? cw : cw & 1;
+  src.tw = (const char *)W.tw + (size_t)st0 * 4 * src.wrow +
+           (size_t)(ct * CT + cwe * 4) * (NW * 4);
+  src.stages = stages;
+  f16v_t acc[MR][2];
+#pragma unroll
+  for (int i = 0; i < MR; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  rd_main<K, CB, MASKED, MR, CW, KP, FR>(acc, smem, src, va, a.dec);
+  const int rows = min(32 * MR, M - m0);
+  const size_t out = (size_t)out_tiles * 16;
+  float *plane = S > 1 ? W.kpart + ((size_t)ks * M + m0) * out : nullptr;
+  rd_end<MR, CW, KP>(acc, smem, rows, [&](int m) { return (size_t)(m0 + m); },
+                     out, ct * COLS, ncols, plane, W.svh, W.y, a.ydt, W.zout);
 }
 
 // ------------------------------------------------------- grouped GEMM

@@ -879,9 +879,10 @@ static hipError_t gemv_scratch(StreamScratch *ss, const int *outs, int count, in
 // Linears ws[0..count) over `rows` rows of the same input: x raw (xdt,
 // prepared in the kernels) or already prepared (f16), to finished outputs
 // ys[i] (ydt) or, with ys null, inner products zs[i] (f16).  Up to 16 rows
-// take the GEMV, one launch per 16 rows for all the linears; wider calls of
-// an integer rate take the GEMM per linear after one prepare launch (other
-// rates take the GEMV 16 rows at a time).
+// take the GEMV, one launch per 16 rows for all the linears; wider calls at
+// the GEMM's rates take the register-decode GEMM for all of them (gemm_rd_takes)
+// or the GEMM per linear after one prepare launch (other rates take the GEMV
+// 16 rows at a time).
 static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *const *pvs, int count,
                               const void *x, int xdt, bool prepared, void *const *ys, int ydt,
                               uint16_t *const *zs, int64_t rows, StreamScratch *ss, hipStream_t s) {
@@ -890,6 +891,38 @@ static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *co
   const size_t xsz = prepared ? 2 : (xdt == exl3::ACT_F32 ? 4 : 2);
   const size_t ysz = ydt == exl3::ACT_F32 ? 4 : 2;
   if (rows > exl3::GEMV_ROWS_MAX && p0->f.gemm_rate()) {
+    // the register-decode GEMM: a prepare of every linear's rows in one
+    // launch, one GEMM launch over them all
+    int outs[4];
+    uintptr_t bits = prepared ? (uintptr_t)x : 0;
+    for (int i = 0; i < count; ++i) {
+      outs[i] = (int)pvs[i]->out;
+      bits |= (uintptr_t)ws[i]->w.data;
+    }
+    if ((bits & 15) == 0 && exl3::gemm_rd_takes(rows, in, outs, count)) {
+      const size_t set = (size_t)rows * in;
+      if (!prepared) {
+        hipError_t e = grow(ss, &ss->xp, &ss->xp_bytes, count * set * 2, s);
+        const uint16_t *suh[4];
+        for (int i = 0; i < count; ++i) suh[i] = (const uint16_t *)ws[i]->scales.data;
+        if (e == hipSuccess)
+          e = exl3::launch_prepare_sets(x, xdt, suh, count, (uint16_t *)ss->xp, (int)rows, in, s);
+        if (e != hipSuccess) return e;
+      }
+      const size_t kpf = exl3::gemm_rd_kpart_floats((int)rows, in, outs, count);
+      if (kpf > 0) {
+        hipError_t e = grow(ss, &ss->kpart, &ss->kpart_bytes, kpf * 4, s);
+        if (e != hipSuccess) return e;
+      }
+      exl3::GemmLinear ls[4];
+      for (int i = 0; i < count; ++i)
+        ls[i] = exl3::GemmLinear{(const uint16_t *)ws[i]->w.data,
+                                 prepared ? (const uint16_t *)x : (const uint16_t *)ss->xp + i * set,
+                                 (const uint16_t *)ws[i]->biases.data, ys ? ys[i] : nullptr,
+                                 zs ? zs[i] : nullptr, outs[i]};
+      return exl3::launch_gemm_rd(ls, count, p0->f, ydt, (int)rows, in, (float *)ss->kpart,
+                                  ss->kpart_bytes / 4, s);
+    }
     for (int i = 0; i < count; ++i) {
       const uint16_t *xp = (const uint16_t *)x;
       if (!prepared) {
@@ -1274,12 +1307,21 @@ exl3_verdict exl3_swiglu(const exl3_weight *gate, const exl3_weight *up, const e
     const WeightPriv *pv2[2] = {pg, pu};
     void *ys[2] = {gu, gu + nel};
     e = run_linears(ws2, pv2, 2, x.data, xdt, false, ys, exl3::ACT_F16, nullptr, rows, ss, s);
-    if (e == hipSuccess) e = exl3::launch_swiglu(gu, gu + nel, gu + 2 * nel, nel, (float)opts->limit, s);
+    // the SwiGLU with down's prepare in its pass where its 16-byte accesses
+    // and 32-bit block count allow (203 rows of 12288: 5.6 + 5.6 -> 6.4 us),
+    // else on its own
+    const bool fuse = ((uintptr_t)down->scales.data & 15) == 0 &&
+                      (uint64_t)rows * (uint64_t)(pd->in / 128) * 16 < (uint64_t)1 << 31;
+    if (e == hipSuccess)
+      e = fuse ? exl3::launch_swiglu_prepare(gu, gu + nel, (const uint16_t *)down->scales.data,
+                                             gu + 2 * nel, (int)rows, (int)pd->in,
+                                             (float)opts->limit, s)
+               : exl3::launch_swiglu(gu, gu + nel, gu + 2 * nel, nel, (float)opts->limit, s);
     const exl3_weight *wd[1] = {down};
     const WeightPriv *pvd[1] = {pd};
     void *yd[1] = {out->data};
     if (e == hipSuccess)
-      e = run_linears(wd, pvd, 1, gu + 2 * nel, exl3::ACT_F16, false, yd, xdt, nullptr, rows, ss, s);
+      e = run_linears(wd, pvd, 1, gu + 2 * nel, exl3::ACT_F16, fuse, yd, xdt, nullptr, rows, ss, s);
     if (e != hipSuccess) {
       if (e == hipErrorInvalidValue) return kShape;
       return hip_failed(e);

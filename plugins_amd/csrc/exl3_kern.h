@@ -2055,6 +2055,27 @@ void moe_gemv_go(const Format &f, int pro, dim3 grid, size_t lds, hipStream_t s,
 }
 
 
+// The dense register-decode GEMM at rate K, or (FR > 0) at the half-integer
+// rate n = 8 FR, in one of its workgroup shapes.
+template <int K, int FR>
+void gemm_rd_go(const Format &f, int shape, dim3 grid, hipStream_t s, const RdArgs &a) {
+  cb_dispatch<FR == 0 ? K : 0>(f, [&](auto CBC, auto MC) {
+    constexpr int CB = decltype(CBC)::value;
+    constexpr bool M = decltype(MC)::value;
+    auto go = [&](auto SH) {
+      constexpr RdShape t = RD_SHAPES[decltype(SH)::value];
+      hipLaunchKernelGGL((gemm_rd_kernel<K, CB, M, t.mr, t.cw, t.kp, FR>), grid,
+                         dim3(rd_threads(t.cw, t.kp)), 0, s, a);
+    };
+    if (shape == 0)
+      go(std::integral_constant<int, 0>{});
+    else if (shape == 1)
+      go(std::integral_constant<int, 1>{});
+    else
+      go(std::integral_constant<int, 2>{});
+  });
+}
+
 // The grouped GEMM over items of up to item_rows slots (RDG_ROWS or half).
 template <int K>
 void gemm_rd_grouped_go(const Format &f, int item_rows, unsigned grid, hipStream_t s,
@@ -2111,6 +2132,8 @@ void gemm_frac_go(const Format &f, dim3 grid, hipStream_t s, const uint32_t *tw,
 #define EXL3_GEMM_GROUPED_GO(KK)                                                             \
   void gemm_grouped_go<KK>(const Format &, dim3, hipStream_t, const uint32_t *, const uint16_t *, \
                            const uint16_t *, void *, int, int, int, const GemmGroup &)
+#define EXL3_GEMM_RD_GO(KK, FR) \
+  void gemm_rd_go<KK, FR>(const Format &, int, dim3, hipStream_t, const RdArgs &)
 #define EXL3_GEMM_RD_GROUPED_GO(KK) \
   void gemm_rd_grouped_go<KK>(const Format &, int, unsigned, hipStream_t, const RdGroupArgs &)
 #define EXL3_GEMM_GO(KK)                                                                    \
@@ -2140,29 +2163,39 @@ EXL3_EXTERN_RATE(8)
 extern template EXL3_GEMM_GO(1);
 extern template EXL3_GEMM_GROUPED_GO(1);
 extern template EXL3_GEMM_RD_GROUPED_GO(1);
+extern template EXL3_GEMM_RD_GO(1, 0);
 extern template EXL3_GEMM_GO(2);
 extern template EXL3_GEMM_GROUPED_GO(2);
 extern template EXL3_GEMM_RD_GROUPED_GO(2);
+extern template EXL3_GEMM_RD_GO(2, 0);
 extern template EXL3_GEMM_GO(3);
 extern template EXL3_GEMM_GROUPED_GO(3);
 extern template EXL3_GEMM_RD_GROUPED_GO(3);
+extern template EXL3_GEMM_RD_GO(3, 0);
 extern template EXL3_GEMM_GO(4);
 extern template EXL3_GEMM_GROUPED_GO(4);
 extern template EXL3_GEMM_RD_GROUPED_GO(4);
+extern template EXL3_GEMM_RD_GO(4, 0);
 extern template EXL3_GEMM_GO(5);
 extern template EXL3_GEMM_GROUPED_GO(5);
 extern template EXL3_GEMM_RD_GROUPED_GO(5);
+extern template EXL3_GEMM_RD_GO(5, 0);
 extern template EXL3_GEMM_GO(6);
 extern template EXL3_GEMM_GROUPED_GO(6);
 extern template EXL3_GEMM_RD_GROUPED_GO(6);
+extern template EXL3_GEMM_RD_GO(6, 0);
 extern template EXL3_GEMM_GO(7);
 extern template EXL3_GEMM_GROUPED_GO(7);
 extern template EXL3_GEMM_RD_GROUPED_GO(7);
+extern template EXL3_GEMM_RD_GO(7, 0);
 extern template EXL3_GEMM_GO(8);
 extern template EXL3_GEMM_GROUPED_GO(8);
 extern template EXL3_GEMM_RD_GROUPED_GO(8);
+extern template EXL3_GEMM_RD_GO(8, 0);
 extern template EXL3_GEMM_FRAC_GO(3);
 extern template EXL3_GEMM_FRAC_GO(5);
+extern template EXL3_GEMM_RD_GO(1, 3);
+extern template EXL3_GEMM_RD_GO(1, 5);
 #endif
 
 }  // namespace exl3

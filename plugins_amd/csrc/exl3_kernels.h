@@ -233,6 +233,29 @@ size_t gemm_kpart_floats(int64_t rows, int in, int out);
 hipError_t launch_gemm(const uint16_t *trellis, const Format &f, const uint16_t *xp,
                        const uint16_t *svh, void *y, int ydt, uint16_t *zout, int rows, int in,
                        int out, float *kpart, size_t kpart_floats, hipStream_t s);
+// The register-decode GEMM (gemm_rate formats): up to four linears that share
+// rows, rate and codebook in one launch, each with its own prepared rows xp
+// f16 [rows, in].
+struct GemmLinear {
+  const uint16_t *trellis;
+  const uint16_t *xp;
+  const uint16_t *svh;
+  void *y;         // finished output in ydt, or null:
+  uint16_t *zout;  // f16(z)
+  int out;
+};
+constexpr int GEMM_RD_MAXW = 4;
+// Whether a call takes it (a rule on the sizes; the trellises and, for rows
+// given prepared, xp must be 16-byte aligned besides), and the split-K plane
+// floats it then needs (0: no split).
+bool gemm_rd_takes(int64_t rows, int in, const int *outs, int count);
+size_t gemm_rd_kpart_floats(int rows, int in, const int *outs, int count);
+hipError_t launch_gemm_rd(const GemmLinear *ls, int count, const Format &f, int ydt, int rows,
+                          int in, float *kpart, size_t kpart_floats, hipStream_t s);
+// prepare with `count` (<= 4) linears' suh in one launch: xp holds count
+// stacked [rows, in] sets.
+hipError_t launch_prepare_sets(const void *x, int xdt, const uint16_t *const *suh, int count,
+                               uint16_t *xp, int rows, int in, hipStream_t s);
 // The split of one GEMV launch over weights of total output width
 // total_out: a linear of width out needs ksplit * rows * out partial floats.
 void gemv_multi_plan(int in, int total_out, bool generic, int rows, int *ksplit, int *tps);

@@ -88,10 +88,15 @@ __global__ __launch_bounds__(64) void finish_kernel(const uint16_t *__restrict__
 // lanes, in had128_pair's stage order and with its sums (lo + hi, lo - hi),
 // so the results are identical.  Block gb of the flattened [rows][in / 128]
 // starts at element 128 gb.  x, suh and xp must be 16-byte aligned.
+struct SuhSets {
+  const uint16_t *p[4];
+};
+// Grid y: one prepared set per consumer (suh sets.p[y], xp stacked).
 __global__ __launch_bounds__(256) void prepare8_kernel(const void *__restrict__ x, int xdt,
-                                                       const uint16_t *__restrict__ suh,
-                                                       uint16_t *__restrict__ xp, int nblk,
-                                                       uint32_t nblocks, int groups) {
+                                                       SuhSets sets, uint16_t *__restrict__ xp0,
+                                                       int nblk, uint32_t nblocks, int groups) {
+  const uint16_t *__restrict__ suh = sets.p[blockIdx.y];
+  uint16_t *__restrict__ xp = xp0 + (size_t)blockIdx.y * nblocks * 128;
   const int j = threadIdx.x & 15;
   const uint32_t gb0 = blockIdx.x * 16u + (threadIdx.x >> 4);
   const bool valid = gb0 < nblocks;  // a 16-lane group is valid or not as a whole
@@ -154,12 +159,38 @@ hipError_t launch_prepare(const void *x, int xdt, const uint16_t *suh, uint16_t 
   const bool aligned = (((uintptr_t)x | (uintptr_t)suh | (uintptr_t)xp) & 15) == 0;
   if (aligned && nblocks * 16 < ((size_t)1 << 31)) {
     hipLaunchKernelGGL(prepare8_kernel, dim3((unsigned)((nblocks + 15) / 16)), dim3(256), 0, s, x,
-                       xdt, suh, xp, nblk, (uint32_t)nblocks, groups);
+                       xdt, SuhSets{{suh, suh, suh, suh}}, xp, nblk, (uint32_t)nblocks, groups);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(prepare_kernel, dim3((nblk + 3) / 4, rows), dim3(256), 0, s, x, xdt, suh, xp,
                      in, nblk, groups);
   return hipGetLastError();
+}
+
+hipError_t launch_prepare_sets(const void *x, int xdt, const uint16_t *const *suh, int count,
+                               uint16_t *xp, int rows, int in, hipStream_t s) {
+  if (rows <= 0 || in <= 0 || in % 128 != 0 || count < 1 || count > 4) return hipErrorInvalidValue;
+  const size_t nblocks = (size_t)rows * (in / 128);
+  uintptr_t bits = (uintptr_t)x | (uintptr_t)xp;
+  SuhSets sets{};
+  for (int i = 0; i < count; ++i) {
+    sets.p[i] = suh[i];
+    bits |= (uintptr_t)suh[i];
+  }
+  if ((bits & 15) == 0 && nblocks * 16 < ((size_t)1 << 31)) {
+    hipLaunchKernelGGL(prepare8_kernel, dim3((unsigned)((nblocks + 15) / 16), count), dim3(256), 0,
+                       s, x, xdt, sets, xp, in / 128, (uint32_t)nblocks, 1);
+    return hipGetLastError();
+  }
+  const size_t xsz = xdt == OUT_F32 ? 4 : 2;
+  for (int i = 0; i < count; ++i)
+    for (int r0 = 0; r0 < rows; r0 += 65535) {
+      const hipError_t e =
+          launch_prepare((const char *)x + (size_t)r0 * in * xsz, xdt, suh[i],
+                         xp + ((size_t)i * rows + r0) * in, std::min(65535, rows - r0), in, s, 1);
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
 }
 
 hipError_t launch_finish(const uint16_t *z, const uint16_t *svh, void *y, int ydt, int rows,
@@ -808,6 +839,153 @@ hipError_t launch_gemm(const uint16_t *trellis, const Format &f, const uint16_t 
   if (sp.splits > 1)
     hipLaunchKernelGGL(gemm_splitk_finish_kernel, dim3(out / 128, (rows + 7) / 8), dim3(512), 0, s,
                        kpart, sp.splits, rows, out, svh, y, ydt, zout);
+  return hipGetLastError();
+}
+
+// ------------------------------------------------- register-decode GEMM
+
+namespace {
+// gemm_splitk_finish_kernel over the launch's linears (column groups side by
+// side in grid x).
+__global__ __launch_bounds__(512) void gemm_rd_finish_kernel(RdArgs a, int S) {
+  const int lane = threadIdx.x & 63;
+  const int m = blockIdx.y * 8 + (threadIdx.x >> 6);
+  if (m >= a.M) return;
+  int wi = 0, c0 = 0;
+#pragma unroll
+  for (int i = 0, c = 0; i < RD_MAXW; ++i) {
+    if (i < a.nw && (int)blockIdx.x >= c) {
+      wi = i;
+      c0 = c;
+    }
+    c += a.w[i].out_tiles / 8;
+  }
+  const RdWeight &W = a.w[wi];
+  const int col = ((int)blockIdx.x - c0) * 128 + 2 * lane;
+  const size_t out = (size_t)W.out_tiles * 16, plane = (size_t)a.M * out, o = (size_t)m * out + col;
+  const float *p = W.kpart + o;
+  float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll 8
+  for (int k = 0; k < S; ++k) {
+    const float2 v = *reinterpret_cast<const float2 *>(p + (size_t)k * plane);
+    s0 += v.x;
+    s1 += v.y;
+  }
+  float v0 = h2f(f2h(s0)), v1 = h2f(f2h(s1));
+  if (W.y == nullptr) {
+    W.zout[o] = f2h(v0);
+    W.zout[o + 1] = f2h(v1);
+    return;
+  }
+  had128_pair(v0, v1, lane);
+  store_out2(W.y, o, f2h(v0 * HAD_SCALE * h2f(W.svh[col])),
+             f2h(v1 * HAD_SCALE * h2f(W.svh[col + 1])), a.ydt);
+}
+
+// Row blocks by the rows (a tile of 128 from 65 on); k-splits to about one
+// workgroup a CU (two and more k-part stages a split), which is what the
+// planes' traffic and the finish launch allow: 4096 -> 12288 at 40 rows in 2 /
+// 4 / 5 / 8 splits 33.9 / 27.0 / 26.2 / 30.8 us.
+struct GemmRdPlan {
+  int shape, ct, mtiles, splits;
+  size_t part_floats;
+};
+GemmRdPlan gemm_rd_plan(int rows, int in, const int *outs, int count) {
+  GemmRdPlan g{};
+  g.shape = rows <= 32 ? 0 : rows <= 64 ? 1 : 2;
+  const RdShape t = RD_SHAPES[g.shape];
+  g.mtiles = (rows + 32 * t.mr - 1) / (32 * t.mr);
+  size_t plane = 0;  // floats of one split
+  for (int i = 0; i < count; ++i) {
+    g.ct += (outs[i] + 64 * t.cw - 1) / (64 * t.cw);
+    plane += (size_t)rows * outs[i];
+  }
+  const int tiles = g.ct * g.mtiles;
+  int S = tiles > 128 ? 1 : std::max(1, std::min(256 / tiles, in / 128 / 4));
+  // planes within the no-alloc matmul's staging beside the call's prepared
+  // rows, whatever scratch the caller has: every entry splits a shape alike
+  const size_t xp = ((size_t)rows * in * 2 + 255) & ~(size_t)255;
+  const size_t stage = NOALLOC_BYTES - NOALLOC_SLOT_BYTES;
+  const size_t room = xp < stage ? stage - xp : 0;
+  while (S > 1 && (size_t)S * plane * 4 > room) --S;
+  g.splits = S;
+  g.part_floats = S > 1 ? (size_t)S * plane : 0;
+  return g;
+}
+}  // namespace
+
+// Against the 256 x 128 tiles (a call, prepare included, K = 4, weights
+// rotated):
+// * one linear: where the weights are large enough for its splits' planes and
+//   its finish launch not to outweigh them, and few row tiles decode them.
+//   4096 -> 12288 at 17 / 40 / 96 / 128 / 256 rows 22.7 / 26.2 / 35.5 / 37.5 /
+//   51.9 us against 35.8 / 33.8 / 38.3 / 42.7 / 46.5; 12288 -> 4096 at 40 / 96
+//   / 128 rows 25.6 / 34.4 / 39.4 against 33.0 / 36.3 / 38.3; 4096 -> 4096 at
+//   17 / 40 / 128 rows 15.9 / 19.9 / 31.5 against 15.6 / 17.0 / 21.9.
+// * several linears, which the other kernel runs one after the other: while
+//   they fill at most 192 of its tiles together.  gate + up (4096 -> 2 x
+//   12288) at 17 / 64 / 128 / 256 / 512 rows 30.0 / 39.4 / 53.1 / 78.0 / 145.8
+//   against 65.6 / 72.2 / 82.3 / 95.0 / 139.7; q + k + v (4096 -> 4096 + 2 x
+//   1024) at 17 / 128 / 1024 rows 17.3 / 30.2 / 82.2 against 39.4 / 55.4 /
+//   117.2; 2048 -> 2 x 6144 at 512 / 1024 rows 48.7 / 92.1 against 69.9 / 89.2.
+bool gemm_rd_takes(int64_t rows, int in, const int *outs, int count) {
+  if (count == 1)
+    return (int64_t)in * outs[0] >= (int64_t)1 << 25 &&
+           (rows <= 96 || (rows <= 128 && outs[0] >= 8192));
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += (outs[i] / 128) * ((rows + 255) / 256);
+  return tiles <= 192 && (uint64_t)rows * in * 2 <= 0xFFFFFFFFull;
+}
+
+size_t gemm_rd_kpart_floats(int rows, int in, const int *outs, int count) {
+  return gemm_rd_plan(rows, in, outs, count).part_floats;
+}
+
+hipError_t launch_gemm_rd(const GemmLinear *ls, int count, const Format &f, int ydt, int rows,
+                          int in, float *kpart, size_t kpart_floats, hipStream_t s) {
+  if (count < 1 || count > GEMM_RD_MAXW || rows < 1 || in <= 0 || in % 128 != 0 ||
+      in / 16 > 65535 || !f.gemm_rate())
+    return hipErrorInvalidValue;
+  // activation offsets (bytes from xp) and a stage's word offsets are 32-bit
+  if ((size_t)rows * in * 2 > 0xFFFFFFFFu) return hipErrorInvalidValue;
+  int outs[GEMM_RD_MAXW], cgs = 0;
+  for (int i = 0; i < count; ++i) {
+    outs[i] = ls[i].out;
+    if (ls[i].out <= 0 || ls[i].out % 128 != 0 || (ls[i].y == nullptr && ls[i].zout == nullptr) ||
+        (((uintptr_t)ls[i].trellis | (uintptr_t)ls[i].xp) & 15) != 0 ||
+        (size_t)4 * (ls[i].out / 16) * f.n * 2 > 0xFFFFFFFFu)
+      return hipErrorInvalidValue;
+    cgs += ls[i].out / 128;
+  }
+  const GemmRdPlan g = gemm_rd_plan(rows, in, outs, count);
+  if (g.mtiles > 65535 || (rows + 7) / 8 > 65535) return hipErrorInvalidValue;
+  if (g.splits > 1 && (kpart == nullptr || kpart_floats < g.part_floats)) return hipErrorInvalidValue;
+  RdArgs a{};
+  a.nw = count;
+  a.ydt = ydt;
+  a.M = rows;
+  a.in_tiles = in / 16;
+  a.dec = f.dec();
+  int ct = 0;
+  for (int i = 0; i < count; ++i) {
+    a.w[i] = RdWeight{reinterpret_cast<const uint32_t *>(ls[i].trellis), ls[i].xp, ls[i].svh,
+                      ls[i].y, ls[i].zout, kpart, ls[i].out / 16, ct};
+    ct += (ls[i].out + 64 * RD_SHAPES[g.shape].cw - 1) / (64 * RD_SHAPES[g.shape].cw);
+    if (g.splits > 1) kpart += (size_t)g.splits * rows * ls[i].out;
+  }
+  const dim3 grid(g.ct, g.mtiles, g.splits);
+  if (f.n == 24)
+    gemm_rd_go<1, 3>(f, g.shape, grid, s, a);
+  else if (f.n == 40)
+    gemm_rd_go<1, 5>(f, g.shape, grid, s, a);
+  else
+    rate_dispatch(f.n / 16, [&](auto KC) {
+      constexpr int K = decltype(KC)::value;
+      if constexpr (K > 0) gemm_rd_go<K, 0>(f, g.shape, grid, s, a);
+    });
+  if (g.splits > 1)
+    hipLaunchKernelGGL(gemm_rd_finish_kernel, dim3(cgs, (rows + 7) / 8), dim3(512), 0, s, a,
+                       g.splits);
   return hipGetLastError();
 }
 

@@ -13,9 +13,12 @@ namespace exl3 {
 template EXL3_GEMM_GO(EXL3_INST_K);
 template EXL3_GEMM_GROUPED_GO(EXL3_INST_K);
 template EXL3_GEMM_RD_GROUPED_GO(EXL3_INST_K);
+template EXL3_GEMM_RD_GO(EXL3_INST_K, 0);
 #else
 template EXL3_GEMM_FRAC_GO(3);
 template EXL3_GEMM_FRAC_GO(5);
+template EXL3_GEMM_RD_GO(1, 3);
+template EXL3_GEMM_RD_GO(1, 5);
 #endif
 
 }  // namespace exl3

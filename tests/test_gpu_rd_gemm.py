@@ -1,0 +1,59 @@
+"""The register-decode GEMM behind exl3_matmul_shared (several linears that
+share their rows): rows on both sides of its row blocks and tiles (32, 64,
+128), widths with a half-empty column tile, inputs of one block and of many
+(split and unsplit k), rates on both sides of its word stages, the half-integer
+rates, each codebook form and output type, against x @ W_public in float64 from
+the oracle's decode; and a large linear alone."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle import oracle as O  # noqa: E402
+from plugins_amd import exl3 as X  # noqa: E402
+from tests import _synth as S  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+FORMS = {"mul1": ("mul1", None, O.CB_MUL1), "mcg": ("mcg", None, O.CB_MCG),
+         "spec1-w15": ("spec1", "spec1-w15", O.spec1(O.TAB_SPEC1_W15)),
+         "pair1": ("pair1", "pair1-w16-v1", O.CB_PAIR1)}
+
+
+def _linear(rng, in_f, out_f, n, form):
+    cb, table, _ = FORMS[form]
+    t, u, v = S.linear(rng, in_f, out_f, n)
+    lin = X.Linear(torch.from_numpy(t.view(np.int16)).to(DEV),
+                   torch.from_numpy(u.view(np.float16)).to(DEV),
+                   torch.from_numpy(v.view(np.float16)).to(DEV), cb, 16, table)
+    return (t, u, v), lin
+
+
+@pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 128, 129, 300])
+@pytest.mark.parametrize("in_f,outs,n,form,dtype", [
+    (128, (128, 384), 64, "mul1", torch.float16), (1024, (640, 128, 256), 48, "mcg", torch.float32),
+    (2176, (256, 128), 128, "mul1", torch.float16), (512, (384, 128, 128, 256), 40, "mul1", torch.float16),
+    (384, (256, 256), 24, "pair1", torch.float16), (640, (128, 256), 112, "spec1-w15", torch.float16)])
+def test_shared_rows_every_linear(rows, in_f, outs, n, form, dtype):
+    rng = np.random.default_rng(rows * 10 + in_f + n)
+    lins = [_linear(rng, in_f, o, n, form) for o in outs]
+    x = S.activations(rng, rows, in_f)
+    ys = X.matmul_shared([lin.weight for _, lin in lins], torch.from_numpy(x).to(DEV).to(dtype))
+    for ((t, u, v), _), o, y in zip(lins, outs, ys):
+        w_inner = O.reconstruct_inner(t, in_f, o, n, FORMS[form][2])
+        want = S.public_matmul(x.astype(np.float64), w_inner, u, v)
+        got = y.float().cpu().numpy()
+        # the repository's bar: three f16 rounding points, 2^-11 each
+        assert S.rel_fro(got, want) < 1e-3
+        assert S.row_rel(got, want).max() < 3e-3
+
+
+def test_large_linear_alone():
+    rng = np.random.default_rng(5)
+    (t, u, v), lin = _linear(rng, 4096, 8192, 32, "mul1")
+    x = S.activations(rng, 97, 4096)
+    for rows in (17, 50, 97):
+        y = lin(torch.from_numpy(x[:rows]).to(DEV)).float().cpu().numpy()
+        want = S.public_matmul(x[:rows].astype(np.float64), O.reconstruct_inner(t, 4096, 8192, 32), u, v)
+        assert S.rel_fro(y, want) < 1e-3
+        assert S.row_rel(y, want).max() < 3e-3
