@@ -151,7 +151,7 @@ SIGNATURES = {
     "exl3_load_bank": (Verdict, [POINTER(LoadCtx), Str, c_uint32, POINTER(Weight)]),
     "exl3_release": (None, [POINTER(Weight)]),
     "exl3_matmul": (Verdict, [POINTER(Weight), Array, c_void_p, POINTER(Array)]),
-    "exl3_matmul_shared": (Verdict, [POINTER(POINTER(Weight)), c_uint32, Array, c_void_p, POINTER(Array)]),
+    "exl3_matmul_shared": (Verdict, [c_void_p, c_uint32, Array, c_void_p, POINTER(Array)]),
     "exl3_moe": (Verdict, [POINTER(Weight), Array, Array, Array, c_bool, c_void_p, POINTER(Array)]),
     "exl3_swiglu": (Verdict, [POINTER(Weight), POINTER(Weight), POINTER(Weight), Array, Array, Array,
                               POINTER(SwigluOpts), c_void_p, POINTER(Array)]),
@@ -232,7 +232,10 @@ def _torch():
     return torch
 
 
-def dtype_of(t) -> int:
+_DTYPES: dict = {}  # torch dtype -> ABI dtype, filled at the first use
+
+
+def _dtype_table() -> dict:
     torch = _torch()
     table = {torch.float16: DT_F16, torch.bfloat16: DT_BF16, torch.float32: DT_F32,
              torch.int16: DT_I16, torch.int32: DT_I32, torch.uint8: DT_U8, torch.int64: DT_I64,
@@ -240,26 +243,29 @@ def dtype_of(t) -> int:
     for name, code in (("uint16", DT_U16), ("uint32", DT_U32)):
         if hasattr(torch, name):
             table[getattr(torch, name)] = code
-    if t.dtype not in table:
+    _DTYPES.update(table)
+    return table
+
+
+def dtype_of(t) -> int:
+    code = (_DTYPES or _dtype_table()).get(t.dtype)
+    if code is None:
         raise TypeError(f"no ABI dtype for {t.dtype}")
-    return table[t.dtype]
+    return code
 
 
 def array(t, dtype: int | None = None) -> Array:
     """An Array descriptor over a contiguous device tensor (None: empty)."""
-    a = Array()
     if t is None:
-        return a
+        return Array()
     if not t.is_contiguous():
         raise ValueError("the ABI takes dense row-major arrays")
-    if t.dim() > MAX_DIMS:
+    shape = tuple(t.shape)
+    if len(shape) > MAX_DIMS:
         raise ValueError("too many dims")
-    a.data = t.data_ptr()
-    a.dtype = dtype_of(t) if dtype is None else dtype
-    a.ndim = t.dim()
-    for i, s in enumerate(t.shape):
-        a.shape[i] = s
-    return a
+    # one constructor call (1.8 us against 2.8 a field at a time: three linears
+    # of 3 rows in one call 20.4 -> 17.6 us, a one-row matmul 11.8 -> 11.2)
+    return Array(t.data_ptr(), dtype_of(t) if dtype is None else dtype, len(shape), shape)
 
 
 def stream_handle(stream=None) -> int:
@@ -449,16 +455,20 @@ def wrap(trellis, suh, svh, codebook: str = "mul1", window: int = 16, device: in
     return w
 
 
+def _out_features(w: Weight) -> int:
+    b = w.biases
+    return b.shape[b.ndim - 1]
+
+
 def _out_tensor(like, last: int, dtype=None):
-    torch = _torch()
-    return torch.empty(*like.shape[:-1], last, dtype=dtype or like.dtype, device=like.device)
+    shape = (*like.shape[:-1], last)
+    return like.new_empty(shape) if dtype is None else like.new_empty(shape, dtype=dtype)
 
 
 def matmul(w: Weight, x, out=None, stream=None):
     """x @ W^T through the library (QuantTable.matmul).  `out` is written if
     given, else allocated with torch (the library never owns it here)."""
-    out_f = w.biases.shape[w.biases.ndim - 1]
-    y = out if out is not None else _out_tensor(x, out_f)
+    y = out if out is not None else _out_tensor(x, _out_features(w))
     a = array(y)
     check(lib().exl3_matmul(ctypes.byref(w), array(x), stream_handle(stream), ctypes.byref(a)),
           "matmul")
@@ -468,8 +478,8 @@ def matmul(w: Weight, x, out=None, stream=None):
 def matmul_shared(ws, x, outs=None, stream=None):
     """Several linears reading the same rows in one launch (outs[i] = x @ W_i^T)."""
     n = len(ws)
-    ptrs = (POINTER(Weight) * n)(*[ctypes.pointer(w) for w in ws])
-    ys = outs if outs is not None else [_out_tensor(x, w.biases.shape[w.biases.ndim - 1]) for w in ws]
+    ptrs = (c_void_p * n)(*map(ctypes.addressof, ws))
+    ys = outs if outs is not None else [_out_tensor(x, _out_features(w)) for w in ws]
     arr = (Array * n)(*[array(y) for y in ys])
     check(lib().exl3_matmul_shared(ptrs, n, array(x), stream_handle(stream), arr), "matmul_shared")
     return ys
