@@ -1894,6 +1894,7 @@ const char *exl3_swiglu_path(const exl3_weight *gate, const exl3_weight *up,
   a.rows = (int)rows;
   a.topk = (int)topk;
   a.experts = (int)std::max<int64_t>(pg->experts, 1);
+  a.inter = (int)pg->out;
   a.inds = reinterpret_cast<const uint32_t *>(&a);  // routed: any non-null
   a.verify_rows = verify_rows;
   a.aligned = (((uintptr_t)gate->w.data | (uintptr_t)up->w.data | (uintptr_t)down->w.data) & 15) == 0;

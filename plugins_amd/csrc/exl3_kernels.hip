@@ -1437,13 +1437,22 @@ constexpr size_t MOE_FUSED_MID_MAX_WG = 2048;
 
 // Grouped GEMMs when the slots average at least this many per expert (and
 // every rate is an integer rate); below, the routed GEMV items, which decode
-// an expert's weights once per 4 slots: 16 experts of 4096 x 2048 at K = 3,
-// 17 / 24 / 32 slots each, 250 / 325 / 470 us a call through the items
-// against 115 / 118 / 122 through the GEMM.  (Calls of up to 16 slots an
-// expert keep the decode chain's sums.)
-constexpr int MOE_GEMM_SLOTS_PER_EXPERT = 17;
-// ... and the average from which a call counts as prefill-sized: swiglu_shared
-// refuses such batches.
+// an expert's weights once per 4 slots.  The fewer workgroups gate + up make
+// (experts x column tiles), the longer the GEMM's unsplit k weighs:
+// * 256 or more: from 4 slots.  K = 3, slots 3 / 4 / 8 / 16 an expert, items
+//   against GEMM: 256 experts of 7168 x 2048 1560 / 1854 / 3199 / 5844 us
+//   against 1486 / 1547 / 1590 / 1689; 128 of 4096 x 1024 265 / 312 / 489 / 879
+//   against 250 / 252 / 260 / 280; 64 of 1024 x 512 (K = 2) 46 / 49 / 63 / 95
+//   against 45 / 47 / 46 / 53.
+// * 64 or more: from 8.  16 of 2048 x 512 (K = 4), 4 / 8 / 16 slots: 46 / 62 /
+//   98 against 55 / 59 / 60.
+// * else from 17 (a handful of workgroups; one decode chain's sums up to there).
+int moe_gemm_slots(const MoeArgs &a) {
+  const long wg = (long)a.experts * 2 * ((a.inter + 64 * RDG_CW - 1) / (64 * RDG_CW));
+  return wg >= 256 ? 4 : wg >= 64 ? 8 : 17;
+}
+// The average from which a call counts as prefill-sized: swiglu_shared refuses
+// such batches.
 constexpr int MOE_PREFILL_SLOTS_PER_EXPERT = 32;
 
 // Grouped GEMM items hold up to 64 slots (32-row blocks by two, four
@@ -1461,7 +1470,7 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 bool moe_uses_gemm(const MoeArgs &a, bool gu_generic, bool d_generic) {
   const long slots = (long)a.rows * a.topk;
   return !gu_generic && !d_generic && a.inds != nullptr && !a.verify_rows && a.aligned &&
-         slots >= (long)MOE_GEMM_SLOTS_PER_EXPERT * a.experts;
+         slots >= (long)moe_gemm_slots(a) * a.experts;
 }
 
 bool moe_prefill_sized(const MoeArgs &a, bool gu_generic, bool d_generic) {

@@ -46,3 +46,26 @@ def test_grouped_gemm_item_edges(counts, n, hidden, inter):
     # the repository's bar: three f16 rounding points a linear, 2^-11 each
     assert S.rel_fro(y, want) < 1e-3
     assert S.row_rel(y, want).max() < 3e-3
+
+
+@pytest.mark.parametrize("E,topk,rows,hidden,inter,path", [
+    (128, 4, 128, 256, 256, "routed-gemm"),   # 256 workgroups, 4 slots an expert
+    (128, 4, 127, 256, 256, "routed-gemv"),
+    (32, 4, 64, 256, 256, "routed-gemm"),     # 64 workgroups, 8 slots
+    (32, 4, 63, 256, 256, "routed-gemv"),
+    (16, 2, 128, 256, 256, "routed-gemv"),    # 32 workgroups, 16 slots
+    (16, 2, 136, 256, 256, "routed-gemm")])
+def test_grouped_gemm_rule(E, topk, rows, hidden, inter, path):
+    rng = np.random.default_rng(E + rows)
+    n = 48
+    gn, g = _bank(rng, E, hidden, inter, n, "mul1")
+    un, u = _bank(rng, E, hidden, inter, n, "mul1")
+    dn, d = _bank(rng, E, inter, hidden, n, "mul1")
+    x = S.activations(rng, rows, hidden)
+    inds, scores = O.route_topk(rng.standard_normal((rows, E)).astype(np.float32), topk)
+    assert X.swiglu_path(g, u, d, rows, topk) == path
+    y = X.swiglu(g, u, d, torch.from_numpy(x).to(DEV), torch.from_numpy(inds).to(DEV),
+                 torch.from_numpy(scores).to(DEV)).float().cpu().numpy()
+    want = O.moe_swiglu(x.astype(np.float32), gn, un, dn, inds, scores, hidden, inter, n)
+    assert S.rel_fro(y, want) < 1e-3
+    assert S.row_rel(y, want).max() < 3e-3
