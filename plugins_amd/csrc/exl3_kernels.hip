@@ -474,11 +474,29 @@ void gemv_plan(int in, int out, int groups, int rows, int *ksplit, int *tps, int
     }
   }
   const int target = rows > 4 ? 256 : 512;
-  int ks = std::min(nb, std::max(1, rows > 4 ? target / cgs : (target + cgs - 1) / cgs));
-  int bps = std::min(tps_max / 8, (nb + ks - 1) / ks);  // blocks per split
-  bps = std::max(bps, (nb + GEMV_KSPLIT_MAX - 1) / GEMV_KSPLIT_MAX);
+  const int ks0 = std::min(nb, std::max(1, rows > 4 ? target / cgs : (target + cgs - 1) / cgs));
+  auto split = [&](int cap, int *ks) {  // blocks per split and splits under a cap
+    int bps = std::min(cap, (nb + ks0 - 1) / ks0);
+    bps = std::max(bps, (nb + GEMV_KSPLIT_MAX - 1) / GEMV_KSPLIT_MAX);
+    *ks = (nb + bps - 1) / bps;
+    return bps;
+  };
+  int bps = split(tps_max / 8, ksplit);
+  if (rows > 4 && groups == 1) {
+    // longer splits, as far as the prepare's passes hold the rows, where they
+    // take less time on the busiest CU: 12288 -> 4096 in 8 splits of 12
+    // blocks, 256 workgroups, against 12 of 8, 384: an MLP of 6 rows 38.4 ->
+    // 36.9 us.  (Two more prepare passes, for 16 rows of 12 blocks, measured
+    // no faster a decode step of 16.)
+    int ks2;
+    const int bps2 = split(std::min(GEMV_TPS_ONE_ROW_MAX / 8, PREP_PASSES * PREP_GROUPS / rows), &ks2);
+    auto cost = [&](int ks, int b) { return (((long)cgs * ks + 255) / 256) * b; };
+    if (bps2 > bps && cost(ks2, bps2) < cost(*ksplit, bps)) {
+      bps = bps2;
+      *ksplit = ks2;
+    }
+  }
   *tps = 8 * bps;
-  *ksplit = (nb + bps - 1) / bps;
 }
 
 int gemv_ksplit(int in, int out, int groups, int rows) {
