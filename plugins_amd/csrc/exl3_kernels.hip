@@ -946,7 +946,9 @@ GemmRdPlan gemm_rd_plan(int rows, int in, const int *outs, int count) {
 //   against 65.6 / 72.2 / 82.3 / 95.0 / 139.7; q + k + v (4096 -> 4096 + 2 x
 //   1024) at 17 / 128 / 1024 rows 17.3 / 30.2 / 82.2 against 39.4 / 55.4 /
 //   117.2; 2048 -> 2 x 6144 at 512 / 1024 rows 48.7 / 92.1 against 69.9 / 89.2.
+// Inputs past its 65535 k-tiles keep the 256 x 128 tiles.
 bool gemm_rd_takes(int64_t rows, int in, const int *outs, int count) {
+  if (in / 16 > 65535) return false;
   if (count == 1)
     return (int64_t)in * outs[0] >= (int64_t)1 << 25 &&
            (rows <= 96 || (rows <= 128 && outs[0] >= 8192));

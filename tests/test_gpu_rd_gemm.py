@@ -57,3 +57,16 @@ def test_large_linear_alone():
         want = S.public_matmul(x[:rows].astype(np.float64), O.reconstruct_inner(t, 4096, 8192, 32), u, v)
         assert S.rel_fro(y, want) < 1e-3
         assert S.row_rel(y, want).max() < 3e-3
+
+
+def test_input_past_its_tile_count():
+    """65536 k-tiles: beyond the register-decode kernel's range, the 256 x 128
+    tiles take the call."""
+    in_f, out_f = 16 * 65536, 128
+    rng = np.random.default_rng(9)
+    (t, u, v), lin = _linear(rng, in_f, out_f, 16, "mul1")
+    x = S.activations(rng, 17, in_f)
+    y = lin(torch.from_numpy(x).to(DEV)).float().cpu().numpy()
+    want = S.public_matmul(x.astype(np.float64), O.reconstruct_inner(t, in_f, out_f, 16), u, v)
+    assert S.rel_fro(y, want) < 1e-3
+    assert S.row_rel(y, want).max() < 3e-3
