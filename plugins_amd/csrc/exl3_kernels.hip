@@ -91,12 +91,17 @@ __global__ __launch_bounds__(64) void finish_kernel(const uint16_t *__restrict__
 struct SuhSets {
   const uint16_t *p[4];
 };
-// Grid y: one prepared set per consumer (suh sets.p[y], xp stacked).
+// SETS: grid y is one prepared set per consumer (suh sets.p[y], xp stacked).
+// Its own instantiation: one set's suh comes preloaded in SGPRs, the sets'
+// pointer from an indexed argument load ahead of suh's own.
+template <bool SETS>
 __global__ __launch_bounds__(256) void prepare8_kernel(const void *__restrict__ x, int xdt,
-                                                       SuhSets sets, uint16_t *__restrict__ xp0,
-                                                       int nblk, uint32_t nblocks, int groups) {
-  const uint16_t *__restrict__ suh = sets.p[blockIdx.y];
-  uint16_t *__restrict__ xp = xp0 + (size_t)blockIdx.y * nblocks * 128;
+                                                       const uint16_t *__restrict__ suh0,
+                                                       uint16_t *__restrict__ xp0, int nblk,
+                                                       uint32_t nblocks, int groups,
+                                                       SuhSets sets) {
+  const uint16_t *__restrict__ suh = SETS ? sets.p[blockIdx.y] : suh0;
+  uint16_t *__restrict__ xp = SETS ? xp0 + (size_t)blockIdx.y * nblocks * 128 : xp0;
   const int j = threadIdx.x & 15;
   const uint32_t gb0 = blockIdx.x * 16u + (threadIdx.x >> 4);
   const bool valid = gb0 < nblocks;  // a 16-lane group is valid or not as a whole
@@ -158,8 +163,8 @@ hipError_t launch_prepare(const void *x, int xdt, const uint16_t *suh, uint16_t 
   const size_t nblocks = (size_t)rows * nblk;
   const bool aligned = (((uintptr_t)x | (uintptr_t)suh | (uintptr_t)xp) & 15) == 0;
   if (aligned && nblocks * 16 < ((size_t)1 << 31)) {
-    hipLaunchKernelGGL(prepare8_kernel, dim3((unsigned)((nblocks + 15) / 16)), dim3(256), 0, s, x,
-                       xdt, SuhSets{{suh, suh, suh, suh}}, xp, nblk, (uint32_t)nblocks, groups);
+    hipLaunchKernelGGL(prepare8_kernel<false>, dim3((unsigned)((nblocks + 15) / 16)), dim3(256), 0,
+                       s, x, xdt, suh, xp, nblk, (uint32_t)nblocks, groups, SuhSets{});
     return hipGetLastError();
   }
   hipLaunchKernelGGL(prepare_kernel, dim3((nblk + 3) / 4, rows), dim3(256), 0, s, x, xdt, suh, xp,
@@ -177,9 +182,10 @@ hipError_t launch_prepare_sets(const void *x, int xdt, const uint16_t *const *su
     sets.p[i] = suh[i];
     bits |= (uintptr_t)suh[i];
   }
+  if (count == 1 && rows <= 65535) return launch_prepare(x, xdt, suh[0], xp, rows, in, s, 1);
   if ((bits & 15) == 0 && nblocks * 16 < ((size_t)1 << 31)) {
-    hipLaunchKernelGGL(prepare8_kernel, dim3((unsigned)((nblocks + 15) / 16), count), dim3(256), 0,
-                       s, x, xdt, sets, xp, in / 128, (uint32_t)nblocks, 1);
+    hipLaunchKernelGGL(prepare8_kernel<true>, dim3((unsigned)((nblocks + 15) / 16), count),
+                       dim3(256), 0, s, x, xdt, suh[0], xp, in / 128, (uint32_t)nblocks, 1, sets);
     return hipGetLastError();
   }
   const size_t xsz = xdt == OUT_F32 ? 4 : 2;
