@@ -882,7 +882,8 @@ static hipError_t gemv_scratch(StreamScratch *ss, const int *outs, int count, in
 // take the GEMV, one launch per 16 rows for all the linears; wider calls at
 // the GEMM's rates take the register-decode GEMM for all of them (gemm_rd_takes)
 // or the GEMM per linear after one prepare launch (other rates take the GEMV
-// 16 rows at a time).
+// 16 rows at a time).  A launch decodes all its linears alike, so linears of
+// different rates or codebooks (an MLP's gate and up) run one by one.
 static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *const *pvs, int count,
                               const void *x, int xdt, bool prepared, void *const *ys, int ydt,
                               uint16_t *const *zs, int64_t rows, StreamScratch *ss, hipStream_t s) {
@@ -890,6 +891,16 @@ static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *co
   const int in = (int)p0->in;
   const size_t xsz = prepared ? 2 : (xdt == exl3::ACT_F32 ? 4 : 2);
   const size_t ysz = ydt == exl3::ACT_F32 ? 4 : 2;
+  bool alike = true;
+  for (int i = 1; i < count; ++i)
+    alike = alike && pvs[i]->f.n == p0->f.n && pvs[i]->f.same_decode(p0->f);
+  if (!alike) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < count && e == hipSuccess; ++i)
+      e = run_linears(ws + i, pvs + i, 1, x, xdt, prepared, ys ? ys + i : nullptr, ydt,
+                      zs ? zs + i : nullptr, rows, ss, s);
+    return e;
+  }
   if (rows > exl3::GEMV_ROWS_MAX && p0->f.gemm_rate()) {
     // the register-decode GEMM: a prepare of every linear's rows in one
     // launch, one GEMM launch over them all
