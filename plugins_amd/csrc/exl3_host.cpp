@@ -1358,8 +1358,17 @@ exl3_verdict exl3_swiglu(const exl3_weight *gate, const exl3_weight *up, const e
   exl3::MoeArgs wa = a;
   wa.rows = (int)std::min<int64_t>(rows, wrows);
   size_t pf = 0;
-  const size_t need =
-      exl3::moe_scratch_bytes(wa, !pg->f.integer_rate(), !pd->f.integer_rate(), &pf);
+  size_t need = exl3::moe_scratch_bytes(wa, !pg->f.integer_rate(), !pd->f.integer_rate(), &pf);
+  if (rows > wrows) {
+    // the last window: few rows may take the GEMV items, whose partial sums a
+    // grouped GEMM's window has no need of
+    exl3::MoeArgs la = a;
+    la.rows = (int)((rows - 1) % wrows + 1);
+    size_t lpf = 0;
+    need = std::max(need, exl3::moe_scratch_bytes(la, !pg->f.integer_rate(),
+                                                  !pd->f.integer_rate(), &lpf));
+    pf = std::max(pf, lpf);
+  }
   hipError_t e = grow(ss, &ss->moe, &ss->moe_bytes, need, s);
   if (e != hipSuccess) return hip_failed(e);
   exl3::Scratch slots;

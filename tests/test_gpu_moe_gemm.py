@@ -69,3 +69,27 @@ def test_grouped_gemm_rule(E, topk, rows, hidden, inter, path):
     want = O.moe_swiglu(x.astype(np.float32), gn, un, dn, inds, scores, hidden, inter, n)
     assert S.rel_fro(y, want) < 1e-3
     assert S.row_rel(y, want).max() < 3e-3
+
+
+def test_last_window_of_few_rows_on_fresh_scratch():
+    """8192 tokens x top-8 run as windows of 8191 rows (the grouped GEMM) and 1
+    row (the GEMV items, which need split-K slots): as the first call on a
+    stream whose scratch is empty."""
+    rng = np.random.default_rng(8192)
+    E, hidden, inter, n, topk, rows = 256, 128, 256, 48, 8, 8192
+    gn, g = _bank(rng, E, hidden, inter, n, "mul1")
+    un, u = _bank(rng, E, hidden, inter, n, "mul1")
+    dn, d = _bank(rng, E, inter, hidden, n, "mul1")
+    x = S.activations(rng, rows, hidden)
+    inds, scores = O.route_topk(rng.standard_normal((rows, E)).astype(np.float32), topk)
+    xd, ids, scs = (torch.from_numpy(a).to(DEV) for a in (x, inds, scores))
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    X.scratch_release(0, stream)
+    y = X.swiglu(g, u, d, xd, ids, scs, stream=stream)
+    stream.synchronize()
+    assert X.stream_status(0, stream).is_ok()
+    at = np.array([0, 4000, 8190, 8191])
+    want = O.moe_swiglu(x[at].astype(np.float32), gn, un, dn, inds[at], scores[at], hidden, inter, n)
+    assert S.rel_fro(y.float().cpu().numpy()[at], want) < 1e-3
+    assert torch.equal(y[-1:], X.swiglu(g, u, d, xd[-1:], ids[-1:], scs[-1:]))
