@@ -379,7 +379,9 @@ exl3_verdict exl3_linear_prepared(const exl3_weight *w, exl3_array xp,
  * every width, so that form is the trellis itself: *out is a borrowed view
  * of it (owned = 0), made without a launch.  Refused when the pieces
  * (opts->rows) would not all take the kernel path (GEMV or GEMM) of the
- * whole call, whose sums are then ordered differently. */
+ * whole call, whose sums are then ordered differently.  Which of the GEMM's
+ * kernels the whole call takes is noted in the view (_pad), and the pieces
+ * take the same: hand it to linear_piece as it is. */
 exl3_verdict exl3_linear_pieces(const exl3_weight *w, const exl3_linear_parts *opts,
                                 exl3_stream s, exl3_array *out);
 

@@ -876,6 +876,19 @@ static hipError_t gemv_scratch(StreamScratch *ss, const int *outs, int count, in
   return hipSuccess;
 }
 
+// Whether a call above 16 rows takes the register-decode GEMM (its word loads
+// are 16 bytes wide).
+static bool takes_rd(const exl3_weight *const *ws, const WeightPriv *const *pvs, int count,
+                     int64_t rows) {
+  int outs[4];
+  uintptr_t bits = 0;
+  for (int i = 0; i < count; ++i) {
+    outs[i] = (int)pvs[i]->out;
+    bits |= (uintptr_t)ws[i]->w.data;
+  }
+  return (bits & 15) == 0 && exl3::gemm_rd_takes(rows, (int)pvs[0]->in, outs, count);
+}
+
 // Linears ws[0..count) over `rows` rows of the same input: x raw (xdt,
 // prepared in the kernels) or already prepared (f16), to finished outputs
 // ys[i] (ydt) or, with ys null, inner products zs[i] (f16).  Up to 16 rows
@@ -884,9 +897,11 @@ static hipError_t gemv_scratch(StreamScratch *ss, const int *outs, int count, in
 // or the GEMM per linear after one prepare launch (other rates take the GEMV
 // 16 rows at a time).  A launch decodes all its linears alike, so linears of
 // different rates or codebooks (an MLP's gate and up) run one by one.
+// tiles: above 16 rows the GEMM of 256 x 128 tiles whatever the sizes.
 static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *const *pvs, int count,
                               const void *x, int xdt, bool prepared, void *const *ys, int ydt,
-                              uint16_t *const *zs, int64_t rows, StreamScratch *ss, hipStream_t s) {
+                              uint16_t *const *zs, int64_t rows, StreamScratch *ss, hipStream_t s,
+                              bool tiles = false) {
   const WeightPriv *p0 = pvs[0];
   const int in = (int)p0->in;
   const size_t xsz = prepared ? 2 : (xdt == exl3::ACT_F32 ? 4 : 2);
@@ -898,20 +913,25 @@ static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *co
     hipError_t e = hipSuccess;
     for (int i = 0; i < count && e == hipSuccess; ++i)
       e = run_linears(ws + i, pvs + i, 1, x, xdt, prepared, ys ? ys + i : nullptr, ydt,
-                      zs ? zs + i : nullptr, rows, ss, s);
+                      zs ? zs + i : nullptr, rows, ss, s, tiles);
     return e;
   }
   if (rows > exl3::GEMV_ROWS_MAX && p0->f.gemm_rate()) {
     // the register-decode GEMM: a prepare of every linear's rows in one
     // launch, one GEMM launch over them all
-    int outs[4];
-    uintptr_t bits = prepared ? (uintptr_t)x : 0;
-    for (int i = 0; i < count; ++i) {
-      outs[i] = (int)pvs[i]->out;
-      bits |= (uintptr_t)ws[i]->w.data;
-    }
-    if ((bits & 15) == 0 && exl3::gemm_rd_takes(rows, in, outs, count)) {
+    if (!tiles && takes_rd(ws, pvs, count, rows)) {
+      int outs[4];
+      for (int i = 0; i < count; ++i) outs[i] = (int)pvs[i]->out;
       const size_t set = (size_t)rows * in;
+      if (prepared && ((uintptr_t)x & 15) != 0) {
+        // its loads are 16 bytes wide: rows that lie otherwise are copied, so
+        // that where they lie does not change the order of their sums
+        hipError_t e = grow(ss, &ss->xp, &ss->xp_bytes, set * 2, s);
+        if (e == hipSuccess)
+          e = hipMemcpyAsync(ss->xp, x, set * 2, hipMemcpyDeviceToDevice, s);
+        if (e != hipSuccess) return e;
+        x = ss->xp;
+      }
       if (!prepared) {
         hipError_t e = grow(ss, &ss->xp, &ss->xp_bytes, count * set * 2, s);
         const uint16_t *suh[4];
@@ -986,11 +1006,11 @@ static hipError_t run_linears(const exl3_weight *const *ws, const WeightPriv *co
 
 static hipError_t run_linear(const exl3_weight *w, const WeightPriv *pv, const void *x, int xdt,
                              bool prepared, void *y, int ydt, uint16_t *zout, int64_t rows,
-                             StreamScratch *ss, hipStream_t s) {
+                             StreamScratch *ss, hipStream_t s, bool tiles = false) {
   void *ys[1] = {y};
   uint16_t *zs[1] = {zout};
   return run_linears(&w, &pv, 1, x, xdt, prepared, y ? ys : nullptr, ydt, zout ? zs : nullptr, rows,
-                     ss, s);
+                     ss, s, tiles);
 }
 
 // A grouped linear (G linears stored as a G-bank): x [..., G, in] ->
@@ -1756,6 +1776,11 @@ exl3_verdict exl3_linear_prepared(const exl3_weight *w, exl3_array xp,
   return ok();
 }
 
+// What linear_pieces notes in its view (_pad) for linear_piece: the whole call
+// takes the GEMM of 256 x 128 tiles, so every piece does (pieces of few rows
+// would take the register-decode GEMM, whose sums are ordered differently).
+constexpr uint32_t PIECES_TILES = 1;
+
 // The kernel path of a call of `rows` rows (run_linears' choice).
 static bool gemm_path(const WeightPriv *pv, int64_t rows) {
   return rows > exl3::GEMV_ROWS_MAX && pv->f.gemm_rate();
@@ -1782,6 +1807,7 @@ exl3_verdict exl3_linear_pieces(const exl3_weight *w, const exl3_linear_parts *o
                     "whole call");
   *out = w->w;  // the packed trellis, borrowed: the pieces' kernels decode it
   out->owned = 0;
+  out->_pad = whole && !takes_rd(&w, &pv, 1, total) ? PIECES_TILES : 0;
   return ok();
 }
 
@@ -1804,7 +1830,7 @@ exl3_verdict exl3_linear_piece(const exl3_weight *w, exl3_array x, const exl3_li
   StreamScratch *ss = scratch_for(pv->device, s);
   std::lock_guard<std::mutex> g(ss->mu);
   hipError_t e = run_linear(w, pv, x.data, xdt, opts->prepared, nullptr, 0, (uint16_t *)out->data,
-                            rows, ss, s);
+                            rows, ss, s, opts->held._pad == PIECES_TILES);
   if (e != hipSuccess) {
     exl3_array_free(out);
     return hip_failed(e);

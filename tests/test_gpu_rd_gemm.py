@@ -70,3 +70,25 @@ def test_input_past_its_tile_count():
     want = S.public_matmul(x.astype(np.float64), O.reconstruct_inner(t, in_f, out_f, 16), u, v)
     assert S.rel_fro(y, want) < 1e-3
     assert S.row_rel(y, want).max() < 3e-3
+
+
+@pytest.mark.parametrize("pieces", [(100, 100), (17, 183), (40, 40), (17, 64, 47), (96, 160)])
+def test_pieces_sum_as_the_whole_call(pieces):
+    """Row pieces on both sides of the register-decode kernel's row rule, and
+    prepared rows that are not 16-byte aligned: the whole call's inner
+    products, bit for bit."""
+    rng = np.random.default_rng(sum(pieces))
+    _, lin = _linear(rng, 4096, 12288, 32, "mul1")
+    x = torch.from_numpy(S.activations(rng, sum(pieces), 4096)).to(DEV)
+    whole = X.linear_split(lin.weight, x, inner=True)
+    v, held = X.linear_pieces(lin.weight, pieces)
+    assert v.is_ok() and held.data == lin.weight.w.data, v
+    xp = X.prepare(lin.weight, x)
+    at = 0
+    for n in pieces:
+        z = X.linear_piece(lin.weight, x[at:at + n], held)
+        assert torch.equal(z, whole[at:at + n])
+        odd = torch.empty(n * 4096 + 1, dtype=torch.float16, device=DEV)[1:].view(n, 4096)
+        odd.copy_(xp[at:at + n])
+        assert torch.equal(X.linear_piece(lin.weight, odd, held, prepared=True), z)
+        at += n
