@@ -293,9 +293,10 @@ struct MoeArgs {
   bool verify_rows;
   bool aligned = true;  // the banks' trellises are 16-byte aligned
 };
-// Whether a routed call takes the grouped GEMM (at least 4, 8 or 17 slots per
-// expert on average, by the workgroups it makes; integer rates, aligned, and
-// not verify_rows) rather than the grouped GEMV's items of up to 4 slots.
+// Whether a routed call takes a grouped GEMM (at least 4, 8 or 17 slots per
+// expert on average, by the workgroups it makes, or 32 of banks that are not
+// aligned; integer rates and not verify_rows) rather than the grouped GEMV's
+// items of up to 4 slots.
 bool moe_uses_gemm(const MoeArgs &a, bool gu_generic, bool d_generic);
 // Whether a call counts as prefill-sized (32 slots per expert on average):
 // swiglu_shared refuses such calls.

@@ -1477,6 +1477,7 @@ struct MoeLayout {
   size_t partial_floats;  // slots in the separate slot buffer: gate, up, down
   int slots, max_items, ks_gu, ks_d, tps_gu, tps_d;
   bool gemm;  // larger expert batches: grouped GEMMs over items of up to RDG_ROWS slots
+              // (banks that are not 16-byte aligned: GM_BM)
   bool direct;  // one row, routes given: every slot its own one-row item
   int item_rows;  // slots an item holds at most
 };
@@ -1518,10 +1519,14 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace
 
+// (Banks that are not 16-byte aligned: the 256-slot grouped GEMM, which reads
+// words by dwords, from prefill-sized averages on.  16 experts of 4096 x 2048
+// at K = 3, 32 / 64 / 300 slots: 237 / 250 / 535 us against 437 / 777 / 3466 in
+// GEMV items.)
 bool moe_uses_gemm(const MoeArgs &a, bool gu_generic, bool d_generic) {
   const long slots = (long)a.rows * a.topk;
-  return !gu_generic && !d_generic && a.inds != nullptr && !a.verify_rows && a.aligned &&
-         slots >= (long)moe_gemm_slots(a) * a.experts;
+  return !gu_generic && !d_generic && a.inds != nullptr && !a.verify_rows &&
+         slots >= (long)(a.aligned ? moe_gemm_slots(a) : MOE_PREFILL_SLOTS_PER_EXPERT) * a.experts;
 }
 
 bool moe_prefill_sized(const MoeArgs &a, bool gu_generic, bool d_generic) {
@@ -1565,8 +1570,10 @@ MoeLayout moe_layout(const MoeArgs &a, bool generic_gu, bool generic_d) {
   // the routes directly (no route launch; a row's routes name distinct
   // experts, and a repeated one would only be read twice)
   L.direct = !L.gemm && a.rows == 1 && a.inds != nullptr;
-  const int item_rows = L.item_rows =
-      !L.gemm ? MOE_ITEM_ROWS : slots < MOE_ITEM64_SLOTS * a.experts ? RDG_ROWS / 2 : RDG_ROWS;
+  const int item_rows = L.item_rows = !L.gemm     ? MOE_ITEM_ROWS
+                                      : !a.aligned ? GM_BM
+                                      : slots < MOE_ITEM64_SLOTS * a.experts ? RDG_ROWS / 2
+                                                                             : RDG_ROWS;
   L.max_items = std::min(a.experts, slots) + (slots + item_rows - 1) / item_rows;
   const int groups = std::max(1, std::min(a.experts, slots));
   moe_plan(a.hidden, a.inter, 2 * groups, L.direct, &L.ks_gu, &L.tps_gu);
@@ -1805,6 +1812,20 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
                        wide);
     auto grouped = [&](const MoeBank *const *b, const uint16_t *const *xp, uint16_t *const *yo,
                        int nw) {
+      if (!a.aligned) {
+        for (int i = 0; i < nw; ++i) {
+          const GemmGroup gg{sorted, items, n_items,
+                             (size_t)(b[i]->in / 16) * (b[i]->out / 16) * (b[i]->f.n / 2), 0, 0};
+          rate_dispatch(b[i]->f.n / 16, [&](auto KC) {
+            constexpr int K = decltype(KC)::value;
+            if constexpr (K > 0)
+              gemm_grouped_go<K>(b[i]->f, dim3(b[i]->out / GM_BN, L.max_items), s,
+                                 reinterpret_cast<const uint32_t *>(b[i]->trellis), xp[i],
+                                 b[i]->svh, yo[i], OUT_F16, b[i]->in / 16, b[i]->out / 16, gg);
+          });
+        }
+        return;
+      }
       RdGroupArgs r{};
       r.nw = nw;
       r.ydt = OUT_F16;

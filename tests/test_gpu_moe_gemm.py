@@ -93,3 +93,41 @@ def test_last_window_of_few_rows_on_fresh_scratch():
     want = O.moe_swiglu(x[at].astype(np.float32), gn, un, dn, inds[at], scores[at], hidden, inter, n)
     assert S.rel_fro(y.float().cpu().numpy()[at], want) < 1e-3
     assert torch.equal(y[-1:], X.swiglu(g, u, d, xd[-1:], ids[-1:], scs[-1:]))
+
+
+def _offset(a, halves):
+    """The array's bits on the device, `halves` 2-byte places past a 16-byte
+    boundary."""
+    flat = torch.from_numpy(np.ascontiguousarray(a).view(np.int16).reshape(-1)).to(DEV)
+    buf = torch.empty(flat.numel() + 8, dtype=torch.int16, device=DEV)
+    view = buf[halves:halves + flat.numel()]
+    view.copy_(flat)
+    return view.view(a.shape)
+
+
+@pytest.mark.parametrize("counts", [(63, 64, 1, 0), (260, 5, 96, 97)])
+@pytest.mark.parametrize("n", [48, 128])
+def test_unaligned_banks_keep_a_grouped_gemm(counts, n):
+    """Trellises at a 4-byte boundary: from 32 slots an expert a grouped GEMM
+    (256-slot items), as the aligned banks."""
+    rng = np.random.default_rng(sum(counts) + n)
+    E, hidden, inter = len(counts), 384, 256
+    inds = np.repeat(np.arange(E, dtype=np.int32), counts)
+    rng.shuffle(inds)
+    rows = inds.size
+    inds = inds.reshape(rows, 1)
+    scores = rng.uniform(0.2, 1.0, (rows, 1)).astype(np.float32)
+    nps, ws = [], []
+    for i, o in ((hidden, inter), (hidden, inter), (inter, hidden)):
+        t, u, v = S.linear(rng, i, o, n, experts=E)
+        nps.append((t, u, v))
+        ws.append(X.wrap(_offset(t, 2), torch.from_numpy(u.view(np.float16)).to(DEV),
+                         torch.from_numpy(v.view(np.float16)).to(DEV)))
+    assert X.swiglu_path(*ws, 32 * E, 1) == "routed-gemm"
+    assert X.swiglu_path(*ws, 32 * E - 1, 1) == "routed-gemv"
+    x = S.activations(rng, rows, hidden)
+    y = X.swiglu(*ws, torch.from_numpy(x).to(DEV), torch.from_numpy(inds).to(DEV),
+                 torch.from_numpy(scores).to(DEV)).float().cpu().numpy()
+    want = O.moe_swiglu(x.astype(np.float32), *nps, inds, scores, hidden, inter, n)
+    assert S.rel_fro(y, want) < 1e-3
+    assert S.row_rel(y, want).max() < 3e-3
