@@ -886,7 +886,7 @@ static bool takes_rd(const exl3_weight *const *ws, const WeightPriv *const *pvs,
     outs[i] = (int)pvs[i]->out;
     bits |= (uintptr_t)ws[i]->w.data;
   }
-  return (bits & 15) == 0 && exl3::gemm_rd_takes(rows, (int)pvs[0]->in, outs, count);
+  return (bits & 15) == 0 && exl3::gemm_rd_takes(rows, (int)pvs[0]->in, outs, count, pvs[0]->f.n);
 }
 
 // Linears ws[0..count) over `rows` rows of the same input: x raw (xdt,

@@ -245,10 +245,10 @@ struct GemmLinear {
   int out;
 };
 constexpr int GEMM_RD_MAXW = 4;
-// Whether a call takes it (a rule on the sizes; the trellises and, for rows
-// given prepared, xp must be 16-byte aligned besides), and the split-K plane
+// Whether a call takes it (a rule on the sizes and the rate n; the trellises
+// must be 16-byte aligned besides), and the split-K plane
 // floats it then needs (0: no split).
-bool gemm_rd_takes(int64_t rows, int in, const int *outs, int count);
+bool gemm_rd_takes(int64_t rows, int in, const int *outs, int count, int n);
 size_t gemm_rd_kpart_floats(int rows, int in, const int *outs, int count);
 hipError_t launch_gemm_rd(const GemmLinear *ls, int count, const Format &f, int ydt, int rows,
                           int in, float *kpart, size_t kpart_floats, hipStream_t s);

@@ -938,29 +938,40 @@ GemmRdPlan gemm_rd_plan(int rows, int in, const int *outs, int count) {
 }
 }  // namespace
 
-// Against the 256 x 128 tiles (a call, prepare included, K = 4, weights
-// rotated):
-// * one linear: where the weights are large enough for its splits' planes and
-//   its finish launch not to outweigh them, and few row tiles decode them.
-//   4096 -> 12288 at 17 / 40 / 96 / 128 / 256 rows 22.7 / 26.2 / 35.5 / 37.5 /
-//   51.9 us against 35.8 / 33.8 / 38.3 / 42.7 / 46.5; 12288 -> 4096 at 40 / 96
-//   / 128 rows 25.6 / 34.4 / 39.4 against 33.0 / 36.3 / 38.3; 4096 -> 4096 at
-//   17 / 40 / 128 rows 15.9 / 19.9 / 31.5 against 15.6 / 17.0 / 21.9.
-// * several linears, which the other kernel runs one after the other: while
-//   they fill at most 192 of its tiles together.  gate + up (4096 -> 2 x
-//   12288) at 17 / 64 / 128 / 256 / 512 rows 30.0 / 39.4 / 53.1 / 78.0 / 145.8
-//   against 65.6 / 72.2 / 82.3 / 95.0 / 139.7; q + k + v (4096 -> 4096 + 2 x
-//   1024) at 17 / 128 / 1024 rows 17.3 / 30.2 / 82.2 against 39.4 / 55.4 /
-//   117.2; 2048 -> 2 x 6144 at 512 / 1024 rows 48.7 / 92.1 against 69.9 / 89.2.
+// Against the 256 x 128 tiles, ratios of a call's time (prepare included,
+// weights rotated), rates n = 16 .. 128 from row to row:
+// * one linear: its splits' planes and its finish launch have to pay, and every
+//   128 rows decode the weights once more, so what counts is in x out.  In x
+//   out = 2^25 (4096 -> 8192, 8192 -> 4096): 17 / 32 / 64 / 96 rows 0.77-0.85 /
+//   0.83-0.93 / 0.97-1.18 / 1.06-1.31; 1.5 x that (4096 -> 12288, 12288 -> 4096):
+//   64 / 65 / 96 / 128 rows 0.81-0.97 / 0.91-1.07 / 0.92-1.09 / 0.92-1.08, above
+//   1.02 at n < 40 (and past 96 rows into 4096); 2 x (4096 -> 16384, 8192 ->
+//   8192): 0.71-0.92 / 0.84-1.03 / 0.84-1.00 / 0.86-1.01; 4 x: at most 0.86.
+// * several linears, which the other kernel runs one after the other: while the
+//   256 x 128 tiles of them all are at most 192 (0.32-0.96; q + k + v of 4096 at
+//   17 / 1024 rows 0.44-0.49 / 0.70-0.75, gate + up of 12288 at 17 / 256 rows
+//   0.47-0.54 / 0.79-0.91; 240 tiles of 3 x 640: 1.06-1.11, 384 of 2 x 12288:
+//   1.04-1.14) and the workgroups here fill the CUs once (128 x 256 tiles: narrow
+//   linears of an odd number of 128 columns waste half a tile; 4 x 128 columns
+//   in 256 / 384 workgroups 0.76-0.80 / 1.03-1.07, 384 + 128 in 240 / 288
+//   0.94-0.96 / 1.25-1.28).  At 7 and 8 bits past 1024 rows to 120 tiles (128
+//   and 136 tiles at 2048 rows: 1.06, 1.03).
 // Inputs past its 65535 k-tiles keep the 256 x 128 tiles.
-bool gemm_rd_takes(int64_t rows, int in, const int *outs, int count) {
+bool gemm_rd_takes(int64_t rows, int in, const int *outs, int count, int n) {
   if (in / 16 > 65535) return false;
-  if (count == 1)
-    return (int64_t)in * outs[0] >= (int64_t)1 << 25 &&
-           (rows <= 96 || (rows <= 128 && outs[0] >= 8192));
-  int64_t tiles = 0;
-  for (int i = 0; i < count; ++i) tiles += (outs[i] / 128) * ((rows + 255) / 256);
-  return tiles <= 192 && (uint64_t)rows * in * 2 <= 0xFFFFFFFFull;
+  if (count == 1) {
+    const int64_t w = (int64_t)in * outs[0], u = (int64_t)1 << 24;
+    if (rows <= 32) return w >= 2 * u;
+    if (rows <= 64) return w >= 3 * u;
+    return rows <= (outs[0] >= 8192 ? 128 : 96) && w >= (n < 40 ? 4 : 3) * u;
+  }
+  int64_t tiles = 0, wgs = 0;
+  for (int i = 0; i < count; ++i) {
+    tiles += (outs[i] / 128) * ((rows + 255) / 256);
+    wgs += ((outs[i] + 255) / 256) * ((rows + 127) / 128);
+  }
+  return tiles <= (n > 96 && rows > 1024 ? 120 : 192) && wgs <= 256 &&
+         (uint64_t)rows * in * 2 <= 0xFFFFFFFFull;
 }
 
 size_t gemm_rd_kpart_floats(int rows, int in, const int *outs, int count) {

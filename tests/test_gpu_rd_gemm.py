@@ -50,11 +50,12 @@ def test_shared_rows_every_linear(rows, in_f, outs, n, form, dtype):
 
 def test_large_linear_alone():
     rng = np.random.default_rng(5)
-    (t, u, v), lin = _linear(rng, 4096, 8192, 32, "mul1")
+    (t, u, v), lin = _linear(rng, 4096, 16384, 32, "mul1")
     x = S.activations(rng, 97, 4096)
+    w_inner = O.reconstruct_inner(t, 4096, 16384, 32)
     for rows in (17, 50, 97):
         y = lin(torch.from_numpy(x[:rows]).to(DEV)).float().cpu().numpy()
-        want = S.public_matmul(x[:rows].astype(np.float64), O.reconstruct_inner(t, 4096, 8192, 32), u, v)
+        want = S.public_matmul(x[:rows].astype(np.float64), w_inner, u, v)
         assert S.rel_fro(y, want) < 1e-3
         assert S.row_rel(y, want).max() < 3e-3
 
@@ -78,7 +79,7 @@ def test_pieces_sum_as_the_whole_call(pieces):
     prepared rows that are not 16-byte aligned: the whole call's inner
     products, bit for bit."""
     rng = np.random.default_rng(sum(pieces))
-    _, lin = _linear(rng, 4096, 12288, 32, "mul1")
+    _, lin = _linear(rng, 4096, 12288, 64, "mul1")
     x = torch.from_numpy(S.activations(rng, sum(pieces), 4096)).to(DEV)
     whole = X.linear_split(lin.weight, x, inner=True)
     v, held = X.linear_pieces(lin.weight, pieces)
@@ -92,3 +93,27 @@ def test_pieces_sum_as_the_whole_call(pieces):
         odd.copy_(xp[at:at + n])
         assert torch.equal(X.linear_piece(lin.weight, odd, held, prepared=True), z)
         at += n
+
+
+def test_rule_of_one_linear():
+    """4096 -> 8192 above 32 rows, where the 256 x 128 tiles are faster, takes
+    them: a call's rows are then those of a 256-row call, bit for bit (the same
+    tiles and k-splits)."""
+    rng = np.random.default_rng(81)
+    _, lin = _linear(rng, 4096, 8192, 48, "mul1")
+    x = torch.from_numpy(S.activations(rng, 256, 4096)).to(DEV)
+    whole = lin(x)
+    for rows in (33, 64, 96, 128):
+        assert torch.equal(lin(x[:rows]), whole[:rows])
+    assert not torch.equal(lin(x[:32]), whole[:32])  # the register-decode kernel
+
+
+@pytest.mark.parametrize("rows,apart", [(10880, False), (11008, True)])
+def test_rule_of_linears_that_share_rows(rows, apart):
+    """128 + 384 columns are 3 half-empty 256-column tiles: one launch up to 256
+    workgroups (85 row tiles), beyond that each linear alone, bit for bit."""
+    rng = np.random.default_rng(82)
+    lins = [_linear(rng, 1024, o, 48, "mul1")[1] for o in (128, 384)]
+    x = torch.from_numpy(S.activations(rng, rows, 1024)).to(DEV)
+    ys = X.matmul_shared([lin.weight for lin in lins], x)
+    assert all(torch.equal(y, lin(x)) for y, lin in zip(ys, lins)) == apart
