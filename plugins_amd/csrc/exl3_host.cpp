@@ -1362,6 +1362,7 @@ exl3_verdict exl3_swiglu(const exl3_weight *gate, const exl3_weight *up, const e
   a.y = out->data;
   a.ydt = xdt;
   a.aligned = (((uintptr_t)gate->w.data | (uintptr_t)up->w.data | (uintptr_t)down->w.data) & 15) == 0;
+  a.n = std::max(pg->f.n, pd->f.n);
   exl3::MoeBank bg{(const uint16_t *)gate->w.data, (const uint16_t *)gate->scales.data,
                    (const uint16_t *)gate->biases.data, pg->f, (int)pg->in, (int)pg->out};
   exl3::MoeBank bu{(const uint16_t *)up->w.data, (const uint16_t *)up->scales.data,
@@ -1940,10 +1941,12 @@ const char *exl3_swiglu_path(const exl3_weight *gate, const exl3_weight *up,
   a.rows = (int)rows;
   a.topk = (int)topk;
   a.experts = (int)std::max<int64_t>(pg->experts, 1);
+  a.hidden = (int)pg->in;
   a.inter = (int)pg->out;
   a.inds = reinterpret_cast<const uint32_t *>(&a);  // routed: any non-null
   a.verify_rows = verify_rows;
   a.aligned = (((uintptr_t)gate->w.data | (uintptr_t)up->w.data | (uintptr_t)down->w.data) & 15) == 0;
+  a.n = std::max(pg->f.n, pd->f.n);
   return exl3::moe_uses_gemm(a, !pg->f.integer_rate(), !pd->f.integer_rate()) ? "routed-gemm"
                                                                               : "routed-gemv";
 }

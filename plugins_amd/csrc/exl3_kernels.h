@@ -292,11 +292,11 @@ struct MoeArgs {
   // (exl3_swiglu_opts.verify_rows)
   bool verify_rows;
   bool aligned = true;  // the banks' trellises are 16-byte aligned
+  int n = 0;            // the largest rate of the banks (halfwords a tile)
 };
-// Whether a routed call takes a grouped GEMM (at least 4, 8 or 17 slots per
-// expert on average, by the workgroups it makes, or 32 of banks that are not
-// aligned; integer rates and not verify_rows) rather than the grouped GEMV's
-// items of up to 4 slots.
+// Whether a routed call takes a grouped GEMM (from 4 to 32 slots per expert on
+// average on, by the banks' sizes; integer rates and not verify_rows) rather
+// than the grouped GEMV's items of up to 4 slots.
 bool moe_uses_gemm(const MoeArgs &a, bool gu_generic, bool d_generic);
 // Whether a call counts as prefill-sized (32 slots per expert on average):
 // swiglu_shared refuses such calls.

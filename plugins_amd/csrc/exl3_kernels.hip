@@ -1487,8 +1487,8 @@ struct MoeLayout {
   size_t sorted, items, n_items, g, u, xd, d, xg, xu, total;
   size_t partial_floats;  // slots in the separate slot buffer: gate, up, down
   int slots, max_items, ks_gu, ks_d, tps_gu, tps_d;
-  bool gemm;  // larger expert batches: grouped GEMMs over items of up to RDG_ROWS slots
-              // (banks that are not 16-byte aligned: GM_BM)
+  bool gemm;  // larger expert batches: grouped GEMMs over items of up to RDG_ROWS slots,
+  bool tiles;  // or the 256-slot ones
   bool direct;  // one row, routes given: every slot its own one-row item
   int item_rows;  // slots an item holds at most
 };
@@ -1497,26 +1497,6 @@ struct MoeLayout {
 // their prepare (measured on the DeepSeek-V3 shape: 1008 workgroups at
 // batch 1 gain ~3 us a call, 8064 at batch 16 lose ~11 us).
 constexpr size_t MOE_FUSED_MID_MAX_WG = 2048;
-
-// Grouped GEMMs when the slots average at least this many per expert (and
-// every rate is an integer rate); below, the routed GEMV items, which decode
-// an expert's weights once per 4 slots.  The fewer workgroups gate + up make
-// (experts x column tiles), the longer the GEMM's unsplit k weighs:
-// * 256 or more: from 4 slots.  K = 3, slots 3 / 4 / 8 / 16 an expert, items
-//   against GEMM: 256 experts of 7168 x 2048 1560 / 1854 / 3199 / 5844 us
-//   against 1486 / 1547 / 1590 / 1689; 128 of 4096 x 1024 265 / 312 / 489 / 879
-//   against 250 / 252 / 260 / 280; 64 of 1024 x 512 (K = 2) 46 / 49 / 63 / 95
-//   against 45 / 47 / 46 / 53.
-// * 64 or more: from 8.  16 of 2048 x 512 (K = 4), 4 / 8 / 16 slots: 46 / 62 /
-//   98 against 55 / 59 / 60.
-// * else from 17 (a handful of workgroups; one decode chain's sums up to there).
-int moe_gemm_slots(const MoeArgs &a) {
-  const long wg = (long)a.experts * 2 * ((a.inter + 64 * RDG_CW - 1) / (64 * RDG_CW));
-  return wg >= 256 ? 4 : wg >= 64 ? 8 : 17;
-}
-// The average from which a call counts as prefill-sized: swiglu_shared refuses
-// such batches.
-constexpr int MOE_PREFILL_SLOTS_PER_EXPERT = 32;
 
 // Grouped GEMM items hold up to 64 slots (32-row blocks by two, four
 // workgroups a CU) below this average of slots per expert, where few experts
@@ -1530,14 +1510,59 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace
 
-// (Banks that are not 16-byte aligned: the 256-slot grouped GEMM, which reads
-// words by dwords, from prefill-sized averages on.  16 experts of 4096 x 2048
-// at K = 3, 32 / 64 / 300 slots: 237 / 250 / 535 us against 437 / 777 / 3466 in
-// GEMV items.)
+namespace {
+// The average of slots an expert from which a call counts as prefill-sized:
+// swiglu_shared refuses such batches.
+constexpr int MOE_PREFILL_SLOTS_PER_EXPERT = 32;
+
+// What a routed call's linears run in: the GEMV items of up to 4 slots, which
+// decode an expert's weights once per item; the register-decode grouped GEMM
+// (items of up to RDG_ROWS slots); or the 256-slot grouped GEMM.
+//
+// Below 32 slots an expert: the items' time goes with the weights they decode
+// (slots / 4 x 3 hidden inter, ~(its millions / 27)^0.65 x 18 us), the GEMM's
+// with its unsplit k, ~21 us + 12.5 ns x (hidden + inter), which is what the
+// quadratic bound follows; and few slots or workgroups (gate + up) leave its row
+// blocks or the CUs empty, which is what the least averages are for.  The GEMM's
+// time over the items' at that edge, K = 3 and 4: 256 experts of 7168 x 2048 at 4
+// slots 0.83, of 1024 x 128 at 5 0.90, 64 of 1024 x 512 at 6 0.91, 32 of 7168 x
+// 512 at 8 0.80, 16 of 2048 x 512 at 8 0.97, 8 of 4096 x 1024 at 12 0.85, 12 of
+// 2048 x 256 at 17 0.72, 8 of 2048 x 512 at 17 0.80; under it 128 of 512 x 128 at
+// 4 1.10, 32 of 1024 x 128 at 8 1.11, 16 of 7168 x 512 at 8 1.22, 8 of 1024 x 128
+// at 31 1.43.  At 7 and 8 bits the GEMM's word loads weigh more (32 of 4096 x 1024
+// at 4 / 6 / 8 slots 1.23 / 1.04 / 0.88).
+//
+// From 32 on the 256-slot GEMM is the other one (0.42-0.95 at 32 and 48 slots).
+// In few workgroups over a short k the finish and the items' second round weigh:
+// 8 experts of 512 x 256 at 64 / 96 / 128 / 200 / 300 slots 1.02 / 1.13 / 1.14 /
+// 1.01 / 0.95, 2 of 1024 x 512 0.93 / 1.07 / 1.15 / 1.03 / 0.97; 2 of 4096 x 2048
+// at 128 slots 0.95-1.01, at 8 bits 1.14.
+//
+// Banks that are not 16-byte aligned: the 256-slot GEMM, which reads words by
+// dwords, from prefill-sized averages on.  16 experts of 4096 x 2048 at K = 3, 32
+// / 64 / 300 slots: 237 / 250 / 535 us against 437 / 777 / 3466 in GEMV items.
+enum class MoeGemm { none, rd, tiles };
+MoeGemm moe_gemm(const MoeArgs &a, bool gu_generic, bool d_generic) {
+  if (gu_generic || d_generic || a.inds == nullptr || a.verify_rows) return MoeGemm::none;
+  const int64_t slots = (int64_t)a.rows * a.topk, E = a.experts;
+  const bool prefill = slots >= MOE_PREFILL_SLOTS_PER_EXPERT * E;
+  if (!a.aligned) return prefill ? MoeGemm::tiles : MoeGemm::none;
+  const int64_t wg = E * 2 * ((a.inter + 64 * RDG_CW - 1) / (64 * RDG_CW));
+  const double k = (double)a.hidden + a.inter;
+  if (prefill)
+    return wg < 64 && (k <= 3072 || a.n > 96) && slots >= 64 * E && slots < 256 * E
+               ? MoeGemm::tiles
+               : MoeGemm::rd;
+  const int least = wg >= 1024 ? 4 : wg >= 512 ? 5 : wg >= 256 ? 6 : wg >= 64 ? 8 : 17;
+  const double work = 0.75 * (double)slots * a.hidden * a.inter;
+  return slots >= least * E && work >= (32e6 + 8.5 * k * k) * (a.n > 96 ? 2.5 : 1.0)
+             ? MoeGemm::rd
+             : MoeGemm::none;
+}
+}  // namespace
+
 bool moe_uses_gemm(const MoeArgs &a, bool gu_generic, bool d_generic) {
-  const long slots = (long)a.rows * a.topk;
-  return !gu_generic && !d_generic && a.inds != nullptr && !a.verify_rows &&
-         slots >= (long)(a.aligned ? moe_gemm_slots(a) : MOE_PREFILL_SLOTS_PER_EXPERT) * a.experts;
+  return moe_gemm(a, gu_generic, d_generic) != MoeGemm::none;
 }
 
 bool moe_prefill_sized(const MoeArgs &a, bool gu_generic, bool d_generic) {
@@ -1576,13 +1601,15 @@ MoeLayout moe_layout(const MoeArgs &a, bool generic_gu, bool generic_d) {
   MoeLayout L{};
   const int slots = a.rows * a.topk;
   L.slots = slots;
-  L.gemm = moe_uses_gemm(a, generic_gu, generic_d);
+  const MoeGemm kind = moe_gemm(a, generic_gu, generic_d);
+  L.gemm = kind != MoeGemm::none;
+  L.tiles = kind == MoeGemm::tiles;
   // one row with its routes given: every slot its own work item, read from
   // the routes directly (no route launch; a row's routes name distinct
   // experts, and a repeated one would only be read twice)
   L.direct = !L.gemm && a.rows == 1 && a.inds != nullptr;
-  const int item_rows = L.item_rows = !L.gemm     ? MOE_ITEM_ROWS
-                                      : !a.aligned ? GM_BM
+  const int item_rows = L.item_rows = !L.gemm   ? MOE_ITEM_ROWS
+                                      : L.tiles ? GM_BM
                                       : slots < MOE_ITEM64_SLOTS * a.experts ? RDG_ROWS / 2
                                                                              : RDG_ROWS;
   L.max_items = std::min(a.experts, slots) + (slots + item_rows - 1) / item_rows;
@@ -1823,7 +1850,7 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
                        wide);
     auto grouped = [&](const MoeBank *const *b, const uint16_t *const *xp, uint16_t *const *yo,
                        int nw) {
-      if (!a.aligned) {
+      if (L.tiles) {
         for (int i = 0; i < nw; ++i) {
           const GemmGroup gg{sorted, items, n_items,
                              (size_t)(b[i]->in / 16) * (b[i]->out / 16) * (b[i]->f.n / 2), 0, 0};

@@ -28,6 +28,9 @@ def _bank(rng, experts, in_f, out_f, n, codebook):
 @pytest.mark.parametrize("n,hidden,inter", [(48, 384, 640), (16, 128, 256), (112, 256, 384),
                                             (128, 512, 128)])
 def test_grouped_gemm_item_edges(counts, n, hidden, inter):
+    # to 64 workgroups and 32 slots an expert: this kernel, its items up to 64
+    # slots; from 48 up to 128
+    counts = counts + 27 * (34 if max(counts) <= 65 else 60,)
     rng = np.random.default_rng(sum(counts) + n)
     E = len(counts)
     inds = np.repeat(np.arange(E, dtype=np.int32), counts)
@@ -49,12 +52,21 @@ def test_grouped_gemm_item_edges(counts, n, hidden, inter):
 
 
 @pytest.mark.parametrize("E,topk,rows,hidden,inter,path", [
-    (128, 4, 128, 256, 256, "routed-gemm"),   # 256 workgroups, 4 slots an expert
-    (128, 4, 127, 256, 256, "routed-gemv"),
-    (32, 4, 64, 256, 256, "routed-gemm"),     # 64 workgroups, 8 slots
-    (32, 4, 63, 256, 256, "routed-gemv"),
-    (16, 2, 128, 256, 256, "routed-gemv"),    # 32 workgroups, 16 slots
-    (16, 2, 136, 256, 256, "routed-gemm")])
+    (512, 4, 512, 256, 256, "routed-gemm"),   # 1024 workgroups, 4 slots an expert
+    (512, 4, 511, 256, 256, "routed-gemv"),
+    (256, 4, 320, 256, 256, "routed-gemm"),   # 512 workgroups, 5 slots
+    (256, 4, 319, 256, 256, "routed-gemv"),
+    (128, 4, 192, 256, 256, "routed-gemm"),   # 256 workgroups, 6 slots
+    (128, 4, 191, 256, 256, "routed-gemv"),
+    (64, 4, 192, 256, 256, "routed-gemm"),    # 128 workgroups, 12 slots: the work's bound
+    (64, 4, 170, 256, 256, "routed-gemv"),
+    (32, 4, 64, 512, 512, "routed-gemm"),     # 128 workgroups, 8 slots
+    (32, 4, 63, 512, 512, "routed-gemv"),
+    (8, 2, 68, 1024, 1024, "routed-gemm"),    # 64 workgroups, 17 slots
+    (16, 2, 255, 128, 256, "routed-gemv"),    # 32 workgroups, no work: to 32 slots
+    (16, 2, 256, 128, 256, "routed-gemm"),
+    (16, 2, 512, 128, 256, "routed-gemm"),    # 64 slots: the 256-slot kernel
+    (16, 2, 2048, 128, 256, "routed-gemm")])
 def test_grouped_gemm_rule(E, topk, rows, hidden, inter, path):
     rng = np.random.default_rng(E + rows)
     n = 48
