@@ -160,9 +160,6 @@ struct GemvCfg {
   int shared_expert;  // routed launches: the index of the shared expert (-1: none)
   int experts;        // routed launches without an item list: expert indices below this
   int routes_k;       // ... > 0: sorted holds k routes, slot k is the shared expert
-  // grouped linears (groups > 0, no item list): item z is linear z of the
-  // G-bank with the call's group_rows rows, whose slots are row * groups + z
-  int groups, group_rows;
   // attention prologue (set: on; the launch's x is then this pointer): the
   // decode attention's per-split slots [rows][attn_nkv][attn_nsplit]
   // [attn_g][128 + 2] (o values, then m, l)
@@ -1777,7 +1774,12 @@ static_assert(MOE_DIRECT_TPS_MAX / 8 <= PREP_GROUPS, "a one-row item's prepare e
 // expert), skipped when not below a.c.experts.  PRO_SWIGLU (down): x is
 // the slots' gate rows and a.c.x2 their up rows (topk 1: row slot), the
 // mid step's SwiGLU and rotation formed in the prepare.  A grouped linear
-// (a.c.groups > 0) takes item z as its linear z over all the call's rows.
+// (items and sorted null) takes item z as its linear z over the call's geo.rows
+// rows, whose slots are row * topk + z (topk: its linears).  geo.rows is also
+// the rows the workgroup's LDS holds (1 without an item list).  All of that
+// comes in preloaded arguments and no instruction of the other launches'
+// waits for it: as two fields of GemvArgs, chosen between in the kernel, it
+// cost every routed launch 1 to 2 % (208 calls of 14 to 70 us).
 template <int K, int CB, bool MASKED, int PRO>
 __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
     const uint32_t *tw0, const uint32_t *tw1, const void *x, uint32_t g0, uint32_t g1,
@@ -1785,22 +1787,22 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
     const MoeItem *__restrict__ items, const uint32_t *__restrict__ n_items, GemvArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int item = blockIdx.z;
+  const GemvGeo geo = GemvGeo::unpack(g0, g1, g2);
   MoeItem it;
   if (items != nullptr) {
     if ((uint32_t)item >= *n_items) return;
     it = items[item];
-  } else if (a.c.groups > 0) {
-    it = MoeItem{(uint32_t)item, 0u, (uint32_t)a.c.group_rows, 0u};
   } else {
-    if ((size_t)item >= a.c.ptotal) return;
-    // uniform across the workgroup; readfirstlane keeps it in a scalar
-    // register for the address arithmetic that follows
-    const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane(
-        a.c.routes_k > 0 && item >= a.c.routes_k ? a.c.shared_expert : (int)sorted[item]);
-    if (e >= (uint32_t)a.c.experts) return;
-    it = MoeItem{e, (uint32_t)item, 1u, 0u};
+    it = MoeItem{(uint32_t)item, (uint32_t)item, (uint32_t)geo.rows, 0u};
+    if (sorted != nullptr) {
+      if ((size_t)item >= a.c.ptotal) return;
+      // uniform across the workgroup; readfirstlane keeps it in a scalar
+      // register for the address arithmetic that follows
+      it.expert = (uint32_t)__builtin_amdgcn_readfirstlane(
+          a.c.routes_k > 0 && item >= a.c.routes_k ? a.c.shared_expert : (int)sorted[item]);
+      if (it.expert >= (uint32_t)a.c.experts) return;
+    }
   }
-  const GemvGeo geo = GemvGeo::unpack(g0, g1, g2);
   const WeightSpan ws = gemv_weight_of(blockIdx.x, geo.cg1, 0, 0, geo.cgend);
   const uint32_t *tw = ws.wi == 0 ? tw0 : tw1;
   const int out_tiles = 8 * (ws.c1 - ws.c0);
@@ -1808,11 +1810,10 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
   GemvRow *ri = reinterpret_cast<GemvRow *>(smem);
   if (threadIdx.x < GEMV_ROWS) {
     const int b = min((int)threadIdx.x, (int)it.count - 1);
-    const int slot = items != nullptr    ? (int)sorted[it.start + b]
-                     : a.c.groups > 0 ? b * a.c.groups + item
-                                      : item;
+    const int slot = items != nullptr ? (int)sorted[it.start + b] : b * topk + item;
     const int in = geo.in_tiles * 16, out = out_tiles * 16;
-    ri[threadIdx.x] = GemvRow{(geo.prepared ? slot : slot / topk) * in, slot * out, slot, 0};
+    ri[threadIdx.x] = GemvRow{(geo.prepared || sorted == nullptr ? slot : slot / topk) * in,
+                              slot * out, slot, 0};
   }
   lds_barrier();
   const RowMap rm{ri, 0, 0};
@@ -1830,9 +1831,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
     gemv_wg<K, CB, MASKED, decltype(P)::value, PRO>(twe, out_tiles, x, geo, a.c, Wx,
                                                sh ? 0 : (int)it.expert, (int)it.count, rm,
                                                blockIdx.x - ws.c0, blockIdx.y, smem + 256,
-                                               items != nullptr    ? MOE_ITEM_ROWS
-                                               : a.c.groups > 0 ? a.c.group_rows
-                                                                : 1);
+                                               geo.rows);
   };
   const int items_n = (int)it.count * (geo.tps / 8);
   if (items_n <= PREP_ITEMS)

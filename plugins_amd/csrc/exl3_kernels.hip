@@ -1658,6 +1658,8 @@ struct MoeGemv {
   bool prepared;
   int pro;
   int in, out, ksplit, tps;
+  int rows = MOE_ITEM_ROWS;  // the rows a workgroup's LDS holds: an item's at most, a
+                             // grouped linear's; 1 where items are single slots
   GemvArgs a;
 };
 
@@ -1666,7 +1668,7 @@ bool moe_geo(const MoeGemv &m, dim3 grid, uint32_t *g0, uint32_t *g1, uint32_t *
   GemvGeo geo{};
   geo.cg1 = m.nweights > 1 ? m.out / 128 : 0;
   geo.cgend = (int)grid.x;
-  geo.rows = MOE_ITEM_ROWS;
+  geo.rows = m.rows;
   geo.xdt = m.xdt;
   geo.prepared = m.prepared ? 1 : 0;
   geo.in_tiles = m.in / 16;
@@ -1758,12 +1760,11 @@ hipError_t launch_gemv_groups(const uint16_t *trellis, const Format &f, const vo
     return hipErrorInvalidValue;
   MoeGemv m = moe_gemv(x, xdt, false, slots, in, out, f, ks, tps);
   m.nweights = 1;
+  m.rows = rows;
   m.a.c.ydt = ydt;
   m.a.c.status = sc.status;
   m.a.c.poll_max = splitk_poll_max();
   m.a.c.drop_partials = splitk_drop();
-  m.a.c.groups = groups;
-  m.a.c.group_rows = rows;
   m.tw[0] = m.tw[1] = reinterpret_cast<const uint32_t *>(trellis);
   GemvWeight &w = m.a.w[0];
   w.suh = suh;
@@ -1774,7 +1775,8 @@ hipError_t launch_gemv_groups(const uint16_t *trellis, const Format &f, const vo
   const dim3 grid(out / 128, ks, groups);
   uint32_t g[3];
   if (!moe_geo(m, grid, &g[0], &g[1], &g[2])) return hipErrorInvalidValue;
-  moe_gemv_launch(f, grid, gemv_lds_bytes(rows, tps, generic), s, m, nullptr, nullptr, nullptr, 1);
+  moe_gemv_launch(f, grid, gemv_lds_bytes(rows, tps, generic), s, m, nullptr, nullptr, nullptr,
+                  groups);
   return hipGetLastError();
 }
 
@@ -1912,6 +1914,8 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
                          : moe_gemv(xd, OUT_F16, true, L.slots, a.inter, a.hidden, down.f, L.ks_d,
                                     L.tps_d);
   md.nweights = 1;
+  const int lds_rows = direct ? 1 : MOE_ITEM_ROWS;
+  mgu.rows = md.rows = lds_rows;
   if (fused_mid) {
     md.pro = PRO_SWIGLU;
     md.a.c.x2 = u;
@@ -1944,7 +1948,6 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
       mgu.a.w[i].sh_svh = sb[i]->svh;
     }
   }
-  const int lds_rows = direct ? 1 : MOE_ITEM_ROWS;
   moe_gemv_launch(gate.f, grid_gu, gemv_lds_bytes(lds_rows, L.tps_gu, gu_generic), s, mgu,
                   isorted, iitems, in_items, a.topk);
   if (!fused_mid)
