@@ -1237,9 +1237,11 @@ void launch_moe_mid(const uint16_t *g, const uint16_t *u, const uint32_t *inds, 
 }
 
 // y[row] = sum_k score * d[slot] (f32, k order), in the output dtype: eight
-// columns a thread, eight slots' loads in flight before their sums (1024 rows
-// x top 8 of 7168: 84 -> 24 us against a column a thread).  wide: y is 16-byte
-// aligned.
+// columns a thread, U slots' loads in flight before their sums (1024 rows x top
+// 8 of 7168: 84 -> 24 us against a column a thread).  U: 2, 4 or 8, the least
+// that holds topk -- the rest of a wider pass is only more instructions (top 2 of
+// 512 columns, 1 row 2.84 us at U = 8, 2.00 at 2; of 4096, 16 rows 3.64 and 3.04).  wide: y is 16-byte aligned.
+template <int U>
 __global__ __launch_bounds__(128) void moe_combine_kernel(const uint16_t *__restrict__ d,
                                                           const uint32_t *__restrict__ inds,
                                                           const void *__restrict__ scores, int sdt,
@@ -1251,19 +1253,19 @@ __global__ __launch_bounds__(128) void moe_combine_kernel(const uint16_t *__rest
   float acc[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) acc[c] = 0.0f;
-  for (int k0 = 0; k0 < topk; k0 += 8) {
-    uint4 v[8];
-    float w[8];
-    bool on[8];
+  for (int k0 = 0; k0 < topk; k0 += U) {
+    uint4 v[U];
+    float w[U];
+    bool on[U];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < U; ++q) {
       const size_t slot = row * topk + min(k0 + q, topk - 1);
       on[q] = k0 + q < topk && (inds ? inds[slot] : 0u) < (uint32_t)experts;
       w[q] = scores ? load_act(scores, slot, sdt) : 1.0f;
       if (on[q]) v[q] = *reinterpret_cast<const uint4 *>(d + slot * hidden + i);
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < U; ++q) {
       if (!on[q]) continue;
       const uint32_t ws[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
 #pragma unroll
@@ -1300,9 +1302,17 @@ __global__ __launch_bounds__(128) void moe_combine_kernel(const uint16_t *__rest
 }
 
 void launch_moe_combine(const MoeArgs &a, const uint16_t *d, hipStream_t s) {
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((a.hidden / 8 + 127) / 128, a.rows), dim3(128), 0, s,
-                     d, a.inds, a.scores, a.sdt, a.topk, a.experts, a.hidden, a.y, a.ydt,
-                     (int)(((uintptr_t)a.y & 15) == 0));
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((a.hidden / 8 + 127) / 128, a.rows), dim3(128), 0, s, d, a.inds,
+                       a.scores, a.sdt, a.topk, a.experts, a.hidden, a.y, a.ydt,
+                       (int)(((uintptr_t)a.y & 15) == 0));
+  };
+  if (a.topk <= 2)
+    go(moe_combine_kernel<2>);
+  else if (a.topk <= 4)
+    go(moe_combine_kernel<4>);
+  else
+    go(moe_combine_kernel<8>);
 }
 
 // The routes of a swiglu with a shared expert (launch_moe_shared_route): one
@@ -1414,6 +1424,8 @@ __global__ __launch_bounds__(64) void moe_shared_route_kernel(
 // Two columns a thread; the slots' loads go out before the gate's chain (logit,
 // exponential, the workgroup's exchange), behind which they went one slot at a
 // time (a DeepSeek-V3-shaped layer at one row 68.8 -> 67.6 us).
+// U as moe_combine_kernel's.
+template <int U>
 __global__ __launch_bounds__(256) void moe_combine_shared_kernel(
     const uint16_t *__restrict__ d, const uint32_t *__restrict__ inds,
     const void *__restrict__ scores, int sdt, int k, int experts,
@@ -1424,7 +1436,6 @@ __global__ __launch_bounds__(256) void moe_combine_shared_kernel(
   const int i = 2 * (blockIdx.x * 256 + threadIdx.x);
   const int ic = min(i, hidden - 2);  // (past the last column: read, not stored)
   const size_t kk = (size_t)k + 1;
-  constexpr int U = 8;
   uint32_t v[U];
   float w[U];
   bool on[U];
@@ -1962,12 +1973,19 @@ hipError_t launch_moe(const MoeArgs &a, const MoeBank &gate, const MoeBank &up,
   }
   moe_gemv_launch(down.f, grid_d, gemv_lds_bytes(lds_rows, L.tps_d, d_generic), s, md,
                   isorted, iitems, in_items, fused_mid ? 1 : a.topk);
-  if (routes_k > 0)
-    hipLaunchKernelGGL(moe_combine_shared_kernel, dim3((a.hidden + 511) / 512, 1), dim3(256), 0,
-                       s, d, a.inds, a.scores, a.sdt, routes_k, a.experts, shared->logit,
-                       shared->gate_vec, a.x, a.xdt, a.hidden, a.y, a.ydt);
-  else
+  auto combine_shared = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((a.hidden + 511) / 512, 1), dim3(256), 0, s, d, a.inds, a.scores,
+                       a.sdt, routes_k, a.experts, shared->logit, shared->gate_vec, a.x, a.xdt,
+                       a.hidden, a.y, a.ydt);
+  };
+  if (routes_k <= 0)
     launch_moe_combine(a, d, s);
+  else if (routes_k <= 2)
+    combine_shared(moe_combine_shared_kernel<2>);
+  else if (routes_k <= 4)
+    combine_shared(moe_combine_shared_kernel<4>);
+  else
+    combine_shared(moe_combine_shared_kernel<8>);
   return hipGetLastError();
 }
 

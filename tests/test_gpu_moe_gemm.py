@@ -143,3 +143,42 @@ def test_unaligned_banks_keep_a_grouped_gemm(counts, n):
     want = O.moe_swiglu(x.astype(np.float32), *nps, inds, scores, hidden, inter, n)
     assert S.rel_fro(y, want) < 1e-3
     assert S.row_rel(y, want).max() < 3e-3
+
+
+@pytest.mark.parametrize("topk", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("rows", [1, 35])
+def test_combine_at_every_width(topk, rows):
+    """The weighted sum's passes of 2, 4 and 8 slots, full and not, a second
+    pass, an out-of-range expert, and y at a 4-byte boundary; and the shared
+    expert's sum beside them."""
+    rng = np.random.default_rng(10 * topk + rows)
+    E, hidden, inter, n = 12, 384, 128, 48
+    gn, g = _bank(rng, E, hidden, inter, n, "mul1")
+    un, u = _bank(rng, E, hidden, inter, n, "mul1")
+    dn, d = _bank(rng, E, inter, hidden, n, "mul1")
+    x = S.activations(rng, rows, hidden)
+    inds, scores = O.route_topk(rng.standard_normal((rows, E)).astype(np.float32), topk)
+    want = O.moe_swiglu(x.astype(np.float32), gn, un, dn, inds, scores, hidden, inter, n)
+    xd, ids, scs = (torch.from_numpy(a).to(DEV) for a in (x, inds, scores))
+    y = X.swiglu(g, u, d, xd, ids, scs)
+    assert S.rel_fro(y.float().cpu().numpy(), want) < 1e-3
+    odd = torch.empty(rows * hidden + 2, dtype=torch.float16, device=DEV)[2:].view(rows, hidden)
+    assert torch.equal(X.swiglu(g, u, d, xd, ids, scs, out=odd), y)
+    if topk > 1:  # the last route names no expert: as with a score of zero
+        ids[:, -1] = E + 1
+        zero = scores.copy()
+        zero[:, -1] = 0.0
+        got = X.swiglu(g, u, d, xd, ids, scs).float().cpu().numpy()
+        want0 = O.moe_swiglu(x.astype(np.float32), gn, un, dn, inds, zero, hidden, inter, n)
+        assert S.rel_fro(got, want0) < 1e-3
+    sn, sw = zip(*(_bank(rng, 1, i, o, n, "mul1") for i, o in ((hidden, inter), (hidden, inter),
+                                                               (inter, hidden))))
+    sw = [X.wrap(*(torch.from_numpy(a[0].view(np.int16 if k == 0 else np.float16)).to(DEV)
+                   for k, a in enumerate(s))) for s in sn]
+    logit = torch.from_numpy(rng.standard_normal(rows).astype(np.float16)).to(DEV)
+    ids = torch.from_numpy(inds).to(DEV)
+    got = X.swiglu_shared(g, u, d, xd, sw, inds=ids, scores=scs, logit=logit).float().cpu().numpy()
+    one = np.zeros((rows, 1), np.int32), np.ones((rows, 1), np.float32)
+    sh = O.moe_swiglu(x.astype(np.float32), *sn, *one, hidden, inter, n)
+    gate = torch.sigmoid(logit).float().cpu().numpy()
+    assert S.rel_fro(got, want + gate[:, None] * sh) < 1e-3
