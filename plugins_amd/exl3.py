@@ -151,7 +151,7 @@ SIGNATURES = {
     "exl3_load_bank": (Verdict, [POINTER(LoadCtx), Str, c_uint32, POINTER(Weight)]),
     "exl3_release": (None, [POINTER(Weight)]),
     "exl3_matmul": (Verdict, [POINTER(Weight), Array, c_void_p, POINTER(Array)]),
-    "exl3_matmul_shared": (Verdict, [c_void_p, c_uint32, Array, c_void_p, POINTER(Array)]),
+    "exl3_matmul_shared": (Verdict, [POINTER(POINTER(Weight)), c_uint32, Array, c_void_p, POINTER(Array)]),
     "exl3_moe": (Verdict, [POINTER(Weight), Array, Array, Array, c_bool, c_void_p, POINTER(Array)]),
     "exl3_swiglu": (Verdict, [POINTER(Weight), POINTER(Weight), POINTER(Weight), Array, Array, Array,
                               POINTER(SwigluOpts), c_void_p, POINTER(Array)]),
@@ -475,13 +475,31 @@ def matmul(w: Weight, x, out=None, stream=None):
     return y
 
 
+_shared = None
+
+
+def _shared_entry():
+    """exl3_matmul_shared taking plain addresses (three pointer objects cost 1.2 us
+    more than checking three weights' type); lib()'s own keeps its signature."""
+    global _shared
+    if _shared is None:
+        fn = lib()["exl3_matmul_shared"]
+        fn.restype, args = SIGNATURES["exl3_matmul_shared"]
+        fn.argtypes = [c_void_p, *args[1:]]
+        _shared = fn
+    return _shared
+
+
 def matmul_shared(ws, x, outs=None, stream=None):
     """Several linears reading the same rows in one launch (outs[i] = x @ W_i^T)."""
     n = len(ws)
+    for w in ws:
+        if not isinstance(w, Weight):
+            raise TypeError("matmul_shared takes Weights")
     ptrs = (c_void_p * n)(*map(ctypes.addressof, ws))
     ys = outs if outs is not None else [_out_tensor(x, _out_features(w)) for w in ws]
     arr = (Array * n)(*[array(y) for y in ys])
-    check(lib().exl3_matmul_shared(ptrs, n, array(x), stream_handle(stream), arr), "matmul_shared")
+    check(_shared_entry()(ptrs, n, array(x), stream_handle(stream), arr), "matmul_shared")
     return ys
 
 

@@ -292,3 +292,24 @@ def test_json_reader_edge_cases():
     assert X.claims('{"quant_method":"exl3",}', cfg) == X.CLAIM_NO
     assert X.claims('[' * 300 + ']' * 300, cfg) == X.CLAIM_NO
     assert X.claims('{"quant_method":"exl3"}', '{"model_type":"deepseek_v41"} x') == X.CLAIM_NO
+
+
+def test_matmul_shared_takes_weights_only():
+    """Neither the mirror nor the entry itself takes another object's address
+    for a weight's."""
+    torch = pytest.importorskip("torch")
+
+    class Stream:
+        cuda_stream = 0
+
+    x = torch.zeros(1, 128, dtype=torch.float16)
+    other = (ctypes.c_char * 4096)()
+    with pytest.raises(TypeError):
+        X.matmul_shared([other], x, outs=[x], stream=Stream)
+    outs = (X.Array * 1)()
+    with pytest.raises(ctypes.ArgumentError):
+        X.lib().exl3_matmul_shared((ctypes.c_void_p * 1)(ctypes.addressof(other)), 1, X.array(x),
+                                   None, outs)
+    # a weight without a handle is the library's to refuse
+    with pytest.raises(X.Exl3Error):
+        X.matmul_shared([X.Weight()], x, outs=[x], stream=Stream)
