@@ -159,7 +159,10 @@ typedef struct exl3_load_ctx {
  * limit > 0 clamps gate to min(g, limit) and up to [-limit, limit] (a NaN
  * passes through).  verify_rows: routed calls take the decode chain (the
  * grouped GEMV items) at any row count, as the reference sends verify rows
- * down its decode chain (sushi_ds41/src/sushi/exl3/root.zig:149). */
+ * down its decode chain (sushi_ds41/src/sushi/exl3/root.zig:149).  Without
+ * it a call takes the grouped GEMM from 4 to 32 slots per expert on average
+ * on (by the banks' sizes; exl3_swiglu_path tells), whose sums are ordered
+ * differently: set it where a batch's rows must run as decode calls do. */
 typedef struct exl3_swiglu_opts {
   uint32_t size;
   int32_t limit;
@@ -654,15 +657,17 @@ void exl3_set_self_check_fault(const char *check);
 /* Library version string and the kernel variant a matmul of `rows` rows
  * takes ("gemv", "gemm"; a grouped linear, `rows` rows per group:
  * "gemm-groups", one prepare and one grouped GEMM launch for every group,
- * or "per-group"): diagnostics for tests and benchmarks. */
+ * "gemv-groups", one GEMV launch for every group, or "per-group"):
+ * diagnostics for tests and benchmarks. */
 const char *exl3_version(void);
 const char *exl3_matmul_path(const exl3_weight *w, int64_t rows);
 
 /* The kernel path a swiglu of `rows` rows takes (topk 0: no routes;
  * verify_rows as exl3_swiglu_opts): "dense-gemv", "dense-gemm",
  * "dense-items", "routed-gemv" (grouped GEMV items of up to 4 slots of one
- * expert) or "routed-gemm" (grouped GEMM over items of up to 256 slots, for
- * prefill-sized expert batches): a diagnostic for tests and benchmarks. */
+ * expert) or "routed-gemm" (grouped GEMM over items of up to 64, 128 or 256
+ * slots, from 4 to 32 slots per expert on average on, by the banks' sizes): a
+ * diagnostic for tests and benchmarks. */
 const char *exl3_swiglu_path(const exl3_weight *gate, const exl3_weight *up,
                              const exl3_weight *down, int64_t rows, int32_t topk,
                              bool verify_rows);

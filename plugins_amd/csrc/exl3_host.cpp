@@ -1013,6 +1013,28 @@ static hipError_t run_linear(const exl3_weight *w, const WeightPriv *pv, const v
                      ss, s, tiles);
 }
 
+// The kernels a grouped linear's call of `rows` rows a group takes: the
+// grouped GEMM over prompt rows at the integer rates, in its kernels' 32-bit
+// offsets; the partial sums of one grouped GEMV launch (0: not that either,
+// each group goes alone) for decode rows and for the rates without a GEMM.
+static bool grouped_gemm(const WeightPriv *pv, int64_t rows) {
+  const int64_t G = pv->groups;
+  return rows > exl3::GEMV_ROWS_MAX && pv->f.integer_rate() &&
+         (uint64_t)(rows * G) * pv->in * 2 <= 0xFFFFFFFFull && G * ((rows + 255) / 256) <= 65535;
+}
+
+static size_t grouped_gemv_floats(const WeightPriv *pv, int64_t rows) {
+  const int64_t G = pv->groups, in = pv->in, out = pv->out;
+  if ((rows > exl3::GEMV_ROWS_MAX && pv->f.gemm_rate()) || G > 65535) return 0;
+  const bool generic = pv->f.gemv_generic();
+  const int wrows = (int)std::min<int64_t>(rows, exl3::GEMV_ROWS_MAX);
+  const int last = (int)((rows - 1) % exl3::GEMV_ROWS_MAX + 1);  // (may split k further)
+  const size_t pf =
+      std::max(exl3::gemv_groups_floats(wrows, (int)G, (int)in, (int)out, generic),
+               exl3::gemv_groups_floats(last, (int)G, (int)in, (int)out, generic));
+  return pf * 4 < (1u << 31) && (int64_t)wrows * G * std::max(in, out) < (int64_t)1 << 31 ? pf : 0;
+}
+
 // A grouped linear (G linears stored as a G-bank): x [..., G, in] ->
 // y [..., G, out], x[..., g, :] through linear g (turboexl3_ds41/plugin.zig:
 // 252-261; sushi_ds41/src/sushi/exl3/linear.zig:24-36).  Prompt rows (above
@@ -1039,8 +1061,7 @@ static exl3_verdict grouped_matmul(const exl3_weight *w, const WeightPriv *pv, e
   StreamScratch *ss = scratch_for(pv->device, s);
   std::lock_guard<std::mutex> lk(ss->mu);
   const int64_t slots = rows * G;
-  if (rows > exl3::GEMV_ROWS_MAX && pv->f.integer_rate() &&
-      (uint64_t)slots * in * 2 <= 0xFFFFFFFFull && G * ((rows + 255) / 256) <= 65535) {
+  if (grouped_gemm(pv, rows)) {
     hipError_t e = grow(ss, &ss->xp, &ss->xp_bytes, (size_t)slots * in * 2, s);
     const int64_t chunk = 65535 - 65535 % G;  // prepare windows of whole rows
     for (int64_t r0 = 0; r0 < slots && e == hipSuccess; r0 += chunk)
@@ -1054,15 +1075,9 @@ static exl3_verdict grouped_matmul(const exl3_weight *w, const WeightPriv *pv, e
     return e == hipSuccess ? ok() : hip_failed(e);
   }
   // decode rows (and prompts at the rates without a GEMM, 16 rows at a time):
-  // every group in one GEMV launch, unless its offsets pass 32 bits
-  const bool generic = pv->f.gemv_generic();
-  const int wrows = (int)std::min<int64_t>(rows, exl3::GEMV_ROWS_MAX);
-  const int last = (int)((rows - 1) % exl3::GEMV_ROWS_MAX + 1);  // (may split k further)
-  const size_t pf = G > 65535 ? 0
-                              : std::max(exl3::gemv_groups_floats(wrows, (int)G, (int)in, (int)outf, generic),
-                                         exl3::gemv_groups_floats(last, (int)G, (int)in, (int)outf, generic));
-  if ((rows <= exl3::GEMV_ROWS_MAX || !pv->f.gemm_rate()) && G <= 65535 && pf * 4 < (1u << 31) &&
-      (int64_t)wrows * G * std::max(in, outf) < (int64_t)1 << 31) {
+  // every group in one GEMV launch
+  const size_t pf = grouped_gemv_floats(pv, rows);
+  if (pf > 0) {
     exl3::Scratch sc;
     hipError_t e = slots_for(ss, pf, s, &sc);
     for (int64_t r0 = 0; r0 < rows && e == hipSuccess; r0 += exl3::GEMV_ROWS_MAX)
@@ -1921,8 +1936,12 @@ const char *exl3_version(void) { return "exl3_mi355x 0.2.0 (gfx950)"; }
 const char *exl3_matmul_path(const exl3_weight *w, int64_t rows) {
   const WeightPriv *pv = priv_of(w);
   if (!pv) return "none";
-  if (pv->groups != 0)  // rows: rows of each group
-    return rows > exl3::GEMV_ROWS_MAX && pv->f.integer_rate() ? "gemm-groups" : "per-group";
+  if (pv->groups != 0) {  // rows: rows of each group
+    if (rows <= 0) return "none";
+    return grouped_gemm(pv, rows)               ? "gemm-groups"
+           : grouped_gemv_floats(pv, rows) > 0 ? "gemv-groups"
+                                               : "per-group";
+  }
   if (rows <= exl3::GEMV_ROWS_MAX) return "gemv";
   return pv->f.gemm_rate() ? "gemm" : "gemv";
 }

@@ -30,6 +30,7 @@ def test_grouped_gemv_every_group(G, in_f, out_f, n, rows, dtype):
     L = X.Loader('{"format":"exl3","codebook":"mul1"}', X.DictSource(src))
     v, w = L.load_tensor("m", in_f)
     assert v.is_ok(), v
+    assert X.matmul_path(w, rows) == "gemv-groups"
     x = torch.from_numpy(S.activations(rng, rows * G, in_f).reshape(rows, G, in_f)).to("cuda").to(dtype)
     y = X.matmul(w, x, out=torch.empty(rows, G, out_f, dtype=dtype, device="cuda"))
     y = y.float().cpu().numpy()
@@ -43,3 +44,25 @@ def test_grouped_gemv_every_group(G, in_f, out_f, n, rows, dtype):
     assert X.stream_status().is_ok()
     X.release(w)
     L.close()
+
+
+def test_path_of_every_width():
+    """One launch over the groups, or each group alone: prompts at a
+    half-integer rate, whose GEMM takes one linear."""
+    rng = np.random.default_rng(3)
+    paths = {}
+    for n in (48, 40, 50):
+        src = {}
+        for g in range(2):
+            t, u, v = S.linear(rng, 256, 128, n)
+            src[f"m.slice.{g}.trellis"] = t.view(np.int16)
+            src[f"m.slice.{g}.suh"] = u.view(np.float16)
+            src[f"m.slice.{g}.svh"] = v.view(np.float16)
+        L = X.Loader('{"format":"exl3","codebook":"mul1"}', X.DictSource(src))
+        v, w = L.load_tensor("m", 256)
+        assert v.is_ok(), v
+        paths[n] = [X.matmul_path(w, r) for r in (1, 16, 17, 300)]
+        X.release(w)
+        L.close()
+    gv, gm = "gemv-groups", "gemm-groups"
+    assert paths == {48: [gv, gv, gm, gm], 40: [gv, gv, "per-group", "per-group"], 50: [gv] * 4}

@@ -120,7 +120,7 @@ def test_grouped_linear(rows):
     v, w = L.load_tensor("m.wo_a", in_f)
     assert v.is_ok(), v
     assert w.flags == 1 and w.w.dims() == (G, in_f // 16, out_f // 16, n)
-    assert X.matmul_path(w, rows) == ("gemm-groups" if rows > 16 else "per-group")
+    assert X.matmul_path(w, rows) == ("gemm-groups" if rows > 16 else "gemv-groups")
     x = S.activations(rng, rows * G, in_f).reshape(rows, G, in_f)
     y = X.matmul(w, dev_f16(x.reshape(rows, G, in_f)), out=torch.empty(rows, G, out_f,
                                                                      dtype=torch.float16, device=DEV))
