@@ -1,8 +1,9 @@
 """The routed experts' grouped GEMM at the edges of its tiles: item sizes on
-both sides of a row block (32), of the tile forms (64, 128) and of an item
-(128), a column tile that is half empty (widths of an odd number of 128-column
-groups), every codebook form's operand path and rates on both sides of the
-word stages' limits, against the oracle's composition."""
+both sides of a row block (32), of the tile forms (64, 128) and of an item (64 or
+128), a column tile that is half empty (widths of an odd number of 128-column
+groups), rates on both sides of the word stages' limits, every codebook form at
+the full and a narrowed window, arrays that are not 16-byte aligned, and the
+rule that chooses it, against the oracle's composition."""
 import numpy as np
 import pytest
 
@@ -182,3 +183,67 @@ def test_combine_at_every_width(topk, rows):
     sh = O.moe_swiglu(x.astype(np.float32), *sn, *one, hidden, inter, n)
     gate = torch.sigmoid(logit).float().cpu().numpy()
     assert S.rel_fro(got, want + gate[:, None] * sh) < 1e-3
+
+
+# codebook, window, table, the oracle's
+FORMS = {"mcg": ("mcg", 16, None, O.CB_MCG), "mcg-w10": ("mcg", 10, None, O.CB_MCG),
+         "mul1-w12": ("mul1", 12, None, O.CB_MUL1),
+         "spec1-w15": ("spec1", 16, "spec1-w15", O.spec1(O.TAB_SPEC1_W15)),
+         "spec1-w9": ("spec1", 9, "spec1-w16", O.spec1(O.TAB_SPEC1_W16)),
+         "pair1": ("pair1", 16, "pair1-w16-v1", O.CB_PAIR1)}
+
+
+@pytest.mark.parametrize("fill", [34, 60])  # items of up to 64 and 128 slots
+@pytest.mark.parametrize("form", FORMS)
+def test_grouped_gemm_codebooks(form, fill):
+    codebook, window, table, ocb = FORMS[form]
+    counts = (33, 64, 5, 130) + 28 * (fill,)
+    rng = np.random.default_rng(fill + len(form))
+    E, hidden, inter, n = len(counts), 256, 384, 48
+    inds = np.repeat(np.arange(E, dtype=np.int32), counts)
+    rng.shuffle(inds)
+    rows = inds.size
+    inds = inds.reshape(rows, 1)
+    scores = rng.uniform(0.2, 1.0, (rows, 1)).astype(np.float32)
+    nps = [S.linear(rng, i, o, n, experts=E)
+           for i, o in ((hidden, inter), (hidden, inter), (inter, hidden))]
+    ws = [X.wrap(torch.from_numpy(t.view(np.int16)).to(DEV), torch.from_numpy(u.view(np.float16)).to(DEV),
+                 torch.from_numpy(v.view(np.float16)).to(DEV), codebook, window, 0, table)
+          for t, u, v in nps]
+    x = S.activations(rng, rows, hidden)
+    assert X.swiglu_path(*ws, rows, 1) == "routed-gemm"
+    y = X.swiglu(*ws, torch.from_numpy(x).to(DEV), torch.from_numpy(inds).to(DEV),
+                 torch.from_numpy(scores).to(DEV)).float().cpu().numpy()
+    want = O.moe_swiglu(x.astype(np.float32), *nps, inds, scores, hidden, inter, n, codebook=ocb,
+                        window=window)
+    assert S.rel_fro(y, want) < 1e-3
+    assert S.row_rel(y, want).max() < 3e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_grouped_gemm_unaligned_arrays(dtype):
+    """x, the scales and y off their 16-byte boundaries: narrower accesses, the
+    same values."""
+    rng = np.random.default_rng(44)
+    E, hidden, inter, n, rows, topk = 32, 256, 384, 48, 300, 4
+    nps = [S.linear(rng, i, o, n, experts=E)
+           for i, o in ((hidden, inter), (hidden, inter), (inter, hidden))]
+
+    def half(a):
+        return torch.from_numpy(a.view(np.float16)).to(DEV)
+
+    trs = [torch.from_numpy(t.view(np.int16)).to(DEV) for t, _, _ in nps]
+    ws = [X.wrap(tr, half(u), half(v)) for tr, (_, u, v) in zip(trs, nps)]
+    odd = [X.wrap(tr, _offset(u, 3).view(torch.float16), _offset(v, 1).view(torch.float16))
+           for tr, (_, u, v) in zip(trs, nps)]
+    x = torch.from_numpy(S.activations(rng, rows, hidden)).to(DEV).to(dtype)
+    inds, scores = O.route_topk(rng.standard_normal((rows, E)).astype(np.float32), topk)
+    ids, scs = torch.from_numpy(inds).to(DEV), torch.from_numpy(scores).to(DEV)
+    assert X.swiglu_path(*ws, rows, topk) == "routed-gemm"
+    y = X.swiglu(*ws, x, ids, scs)
+    xo, yo = (torch.empty(x.numel() + 1, dtype=dtype, device=DEV)[1:].view(x.shape) for _ in range(2))
+    xo.copy_(x)
+    assert torch.equal(X.swiglu(*odd, xo, ids, scs, out=yo), y)
+    want = O.moe_swiglu(x.float().cpu().numpy(), *nps, inds, scores, hidden, inter, n)
+    # beside the bar a bf16 output's own rounding (2^-9)
+    assert S.rel_fro(y.float().cpu().numpy(), want) < (3e-3 if dtype == torch.bfloat16 else 1e-3)

@@ -2,8 +2,9 @@
 share their rows): rows on both sides of its row blocks and tiles (32, 64,
 128), widths with a half-empty column tile, inputs of one block and of many
 (split and unsplit k), rates on both sides of its word stages, the half-integer
-rates, each codebook form and output type, against x @ W_public in float64 from
-the oracle's decode; and a large linear alone."""
+rates, each codebook form, output type and a narrowed window, outputs that are
+not 16-byte aligned, against x @ W_public in float64 from the oracle's decode; a
+large linear alone; and the rules that choose the kernel."""
 import numpy as np
 import pytest
 
@@ -46,6 +47,29 @@ def test_shared_rows_every_linear(rows, in_f, outs, n, form, dtype):
         # the repository's bar: three f16 rounding points, 2^-11 each
         assert S.rel_fro(got, want) < 1e-3
         assert S.row_rel(got, want).max() < 3e-3
+
+
+@pytest.mark.parametrize("rows", [40, 4000])  # k split, and not
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_output_types_and_alignment(rows, dtype):
+    rng = np.random.default_rng(rows)
+    in_f, outs, n, window = 256, (640, 128, 256), 48, 12
+    nps = [S.linear(rng, in_f, o, n) for o in outs]
+    ws = [X.wrap(torch.from_numpy(t.view(np.int16)).to(DEV), torch.from_numpy(u.view(np.float16)).to(DEV),
+                 torch.from_numpy(v.view(np.float16)).to(DEV), "mul1", window) for t, u, v in nps]
+    x = torch.from_numpy(S.activations(rng, rows, in_f)).to(DEV).to(dtype)
+    ys = X.matmul_shared(ws, x)
+    odd = [torch.empty(rows * o + 1, dtype=dtype, device=DEV)[1:].view(rows, o) for o in outs]
+    X.matmul_shared(ws, x, outs=odd)
+    for (t, u, v), o, y, z in zip(nps, outs, ys, odd):
+        assert torch.equal(y, z)
+        w_inner = O.reconstruct_inner(t, in_f, o, n, O.CB_MUL1, window)
+        want = S.public_matmul(x.double().cpu().numpy(), w_inner, u, v)
+        got = y.float().cpu().numpy()
+        # the repository's bar, and a bf16 output's own rounding (2^-9) beside it
+        bar = 3e-3 if dtype == torch.bfloat16 else 1e-3
+        assert S.rel_fro(got, want) < bar
+        assert S.row_rel(got, want).max() < 3 * bar
 
 
 def test_large_linear_alone():

@@ -7,9 +7,9 @@ batches up to 2048 tokens (16384 slots):
 
 * moe_route_kernel: per-expert counts, the slots sorted by expert (exclusive
   scan offsets), work items of at most `item_rows` slots of one expert;
-* gemm_grouped_kernel: the activation rows it gathers (the direct LDS loads'
-  32-bit byte offsets), the trellis words its decode waves read, the output
-  rows it scatters to;
+* gemm_rd_grouped_kernel (aligned banks) and gemm_grouped_kernel (others): the
+  activation rows they gather (the direct LDS loads' 32-bit byte offsets), the
+  trellis words they read, the output rows they scatter to;
 * moe_gemv_kernel: the rows, outputs and partial-sum slots of its items.
 
 Every address is checked against the size of the buffer it indexes, as
@@ -90,6 +90,45 @@ def check_grouped_gemm(sorted_slots, items, slots, in_f, out_f, n, experts):
     return max_act, max_tw, max_out
 
 
+def check_rd_grouped(sorted_slots, items, slots, in_f, out_f, n, experts, item_rows):
+    """gemm_rd_grouped_kernel over every item (rd_group_tile's row forms of 32, 64
+    and 128): as check_grouped_gemm."""
+    in_tiles, out_tiles = in_f // 16, out_f // 16
+    nw = 8 * (n // 16)                      # dwords of a tile
+    wi = (nw * 4 + 63) // 64                # word loads a wave makes a stage
+    stages = in_tiles // 4
+    expert_words = in_tiles * out_tiles * n // 2
+    wrow = out_tiles * nw * 4               # bytes of a k-tile row
+    lane = np.arange(64)
+    max_act = max_tw = max_out = 0
+    for (e, start, M) in items:
+        assert 1 <= M <= item_rows and start + M <= len(sorted_slots)
+        mr = 4 if item_rows > 64 and M > 64 else 2 if M > 32 else 1
+        assert M <= 32 * mr
+        for cw in range(4):
+            for u in range(mr):             # NA = 4 MR / CW loads of 8 rows
+                R = 8 * (mr * cw + u) + (lane >> 3)
+                q = (lane & 7) ^ ((R >> 1) & 7)
+                va = (sorted_slots[start + np.minimum(R, M - 1)] * in_f + 8 * q) * 2
+                assert va.max() < 2 ** 32, "32-bit activation offset overflows"
+                max_act = max(max_act, int(va.max()) + (stages - 1) * 128 + 16)
+        tiles = -(-out_f // 256)
+        for ct in (0, tiles - 1):
+            ncols = min(256, out_f - 256 * ct)
+            for cw in range(4):
+                cwe = cw if 64 * cw < ncols else cw & 1
+                base = e * expert_words * 4 + (ct * 16 + cwe * 4) * nw * 4
+                p = np.minimum(64 * np.arange(wi)[:, None] + lane, 4 * nw - 1)
+                vw = (p // nw) * wrow + (p % nw) * 16
+                last = base + (stages - 1) * 4 * wrow + int(vw.max()) + 16
+                assert last <= (e + 1) * expert_words * 4, "words past the expert's"
+                max_tw = max(max_tw, last)
+            max_out = max(max_out, int(sorted_slots[start:start + M].max()) * out_f + 256 * ct + ncols - 1)
+    assert max_act <= slots * in_f * 2
+    assert max_tw <= experts * expert_words * 4
+    assert max_out < slots * out_f
+
+
 def routings(rng, tokens):
     probs = rng.standard_normal((tokens, E))
     top = np.argsort(-probs, axis=1)[:, :TOPK].astype(np.int32)
@@ -118,6 +157,27 @@ def test_grouped_gemm_indices_deepseek_v3(tokens):
         # row per slot); down: 2048 -> 7168 on xd (one row per slot)
         check_grouped_gemm(sorted_slots, items, slots, HIDDEN, INTER, 16 * K, E)
         check_grouped_gemm(sorted_slots, items, slots, INTER, HIDDEN, 16 * K, E)
+
+
+@pytest.mark.parametrize("tokens,item_rows", [(256, 64), (1024, 64), (2048, 128)])
+def test_rd_grouped_gemm_indices_deepseek_v3(tokens, item_rows):
+    rng = np.random.default_rng(tokens + item_rows)
+    slots = tokens * TOPK
+    for name, inds in routings(rng, tokens):
+        sorted_slots, items, _ = route(inds, E, item_rows)
+        assert len(items) <= max_items(E, slots, item_rows), name
+        check_rd_grouped(sorted_slots, items, slots, HIDDEN, INTER, 16 * K, E, item_rows)
+        check_rd_grouped(sorted_slots, items, slots, INTER, HIDDEN, 16 * K, E, item_rows)
+
+
+@pytest.mark.parametrize("n,hidden,inter", [(16, 128, 256), (112, 256, 384), (128, 512, 128), (48, 384, 640)])
+def test_rd_grouped_gemm_indices_half_tiles(n, hidden, inter):
+    rng = np.random.default_rng(n)
+    inds = rng.integers(0, 40, 2000).reshape(1000, 2)
+    for item_rows in (64, 128):
+        sorted_slots, items, _ = route(inds, 32, item_rows)
+        check_rd_grouped(sorted_slots, items, 2000, hidden, inter, n, 32, item_rows)
+        check_rd_grouped(sorted_slots, items, 2000, inter, hidden, n, 32, item_rows)
 
 
 @pytest.mark.parametrize("tokens", [1, 16, 64, 2048])
