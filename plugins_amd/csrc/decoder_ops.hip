@@ -74,7 +74,6 @@ constexpr int RN_PER = 2;  // 8-element pieces per thread: rows up to 8192
 struct PrepTo {
   const uint16_t *suh[4];
   uint16_t *xp;
-  int count;
 };
 
 template <bool PREP>
@@ -753,7 +752,6 @@ hipError_t launch_rmsnorm_prepare(const float *h, const uint16_t *w, int B, int 
     pt.suh[c] = suh[c];
   }
   pt.xp = xp;
-  pt.count = count;
   hipLaunchKernelGGL(add_rmsnorm_kernel<true>, dim3(B, count), dim3(RN_THREADS), 0, s,
                      const_cast<float *>(h), nullptr, w, nullptr, H, eps, pt);
   return hipGetLastError();

@@ -23,10 +23,14 @@ namespace exl3 {
 // barrier a stage: the activations (shared by the CW waves of a k-part) a
 // stage ahead, the words (one wave's own) two.
 //
-// What bounds it: issue slots.  A decoded weight costs ~3.5 VALU instructions
-// a wave (mul1) however many rows use it, an MFMA 32 matrix cycles and about
-// two VALU slots, so the decode outweighs the MFMAs below 128 rows and is
-// half of them at 256.
+// What bounds it: issue slots.  A decoded weight costs ~4 VALU instructions a
+// wave (mul1, the whole kernel's) however many rows use it, an MFMA 32 matrix
+// cycles, so the decode outweighs the MFMAs up to 64 rows and equals them at
+// 128.  Of the SIMDs' busy cycles VALU instructions issue in 90 % and MFMAs run
+// in 32 % for routed experts of 32 slots each (256 of 7168 x 2048, K = 3, gate +
+// up); in 45 and 35 % for 4096 -> 2 x 12288 at 203 rows, 43 and 17 % for 4096 ->
+// 12288 at 40, whose single round of workgroups waits for its first data and
+// its finish.
 constexpr int RD_BK = 64;
 // The dense GEMM's workgroup shapes (gemm_rd_plan chooses).
 struct RdShape {
@@ -64,11 +68,12 @@ __host__ __device__ constexpr int rd_lds_bytes() {
   return main > fin ? main : fin;
 }
 // Waves a SIMD the registers are budgeted for: four where the accumulators
-// leave it (MR <= 2), two at MR 4, one at 8; fewer where the workgroups' LDS
-// allows fewer.
+// leave it (MR <= 2), two at MR 4; fewer where the workgroups' LDS allows
+// fewer.
 template <int K, int FR, int MR, int CW, int KP>
 __host__ __device__ constexpr int rd_waves() {
-  const int regs = MR <= 2 ? 4 : MR <= 4 ? 2 : 1, wg = CW * KP / 4;  // wg: waves a SIMD each
+  static_assert(MR <= 4, "two waves a SIMD hold the accumulators");
+  const int regs = MR <= 2 ? 4 : 2, wg = CW * KP / 4;  // wg: waves a SIMD each
   const int lds = 160 * 1024 / rd_lds_bytes<K, FR, MR, CW, KP>() * wg;
   return lds < regs ? lds : regs;
 }
@@ -608,8 +613,8 @@ constexpr int RDG_CW = 4, RDG_ROWS = 128;
 // two weights (gate and up) side by side in the column tiles.  A launch's
 // items hold up to 32 MRMAX slots (2: four workgroups a CU, 4: two).
 //
-// Against a workgroup of 256 rows x 128 columns whose eight decode waves fill
-// LDS for eight MFMA waves (what ran before), on 256 experts of 7168 x 2048 at
+// Against gemm_grouped_kernel's workgroup of 256 rows x 128 columns, whose eight
+// decode waves fill LDS for eight MFMA waves, on 256 experts of 7168 x 2048 at
 // K = 3 with 32 slots each (moe layer of 1024 tokens): gate + up 3380 -> 1220
 // us, down 1990 -> 665 us, which is 2.3 and 2.1 TB/s of packed words; 16
 // experts of 4096 x 2048 with 128 / 1024 slots each, the whole call, 273 ->
@@ -632,10 +637,10 @@ struct RdGroupArgs {
   const uint32_t *n_items;
 };
 
-template <int K, int CB, bool MASKED, int MR, int FR>
+template <int K, int CB, bool MASKED, int MR>
 __device__ __forceinline__ void rd_group_tile(const RdGroupArgs &a, const RdGroupWeight &W, int ct,
                                               const MoeItem &item, char *smem) {
-  constexpr int CW = RDG_CW, COLS = 64 * CW, NA = 4 * MR / CW, NW = rd_nw<K, FR>();
+  constexpr int CW = RDG_CW, COLS = 64 * CW, NA = 4 * MR / CW, NW = rd_nw<K, 0>();
   const int lane = threadIdx.x & 63;
   const int cw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int M = (int)item.count, in = a.in_tiles * 16, out_tiles = W.out_tiles;
@@ -662,7 +667,7 @@ __device__ __forceinline__ void rd_group_tile(const RdGroupArgs &a, const RdGrou
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  rd_main<K, CB, MASKED, MR, CW, 1, FR>(acc, smem, src, va, a.dec);
+  rd_main<K, CB, MASKED, MR, CW, 1, 0>(acc, smem, src, va, a.dec);
   const size_t out = (size_t)out_tiles * 16;
   rd_end<MR, CW, 1>(acc, smem, M, [&](int m) { return (size_t)slot_of(m); }, out, ct * COLS, ncols,
                     nullptr, W.svh + (size_t)item.expert * out, W.y, a.ydt, nullptr);
@@ -685,14 +690,14 @@ gemm_rd_grouped_kernel(RdGroupArgs a) {
   // the row blocks that hold the item (1, 2 or 4)
   if constexpr (MRMAX > 2) {
     if ((int)item.count > 64) {
-      rd_group_tile<K, CB, MASKED, 4, 0>(a, W, ct, item, smem);
+      rd_group_tile<K, CB, MASKED, 4>(a, W, ct, item, smem);
       return;
     }
   }
   if ((int)item.count > 32)
-    rd_group_tile<K, CB, MASKED, 2, 0>(a, W, ct, item, smem);
+    rd_group_tile<K, CB, MASKED, 2>(a, W, ct, item, smem);
   else
-    rd_group_tile<K, CB, MASKED, 1, 0>(a, W, ct, item, smem);
+    rd_group_tile<K, CB, MASKED, 1>(a, W, ct, item, smem);
 }
 
 }  // namespace exl3

@@ -1166,7 +1166,9 @@ exl3_verdict exl3_matmul_noalloc(const exl3_weight *w, exl3_array x, exl3_stream
   if (out.dtype != x.dtype || out.ndim < 1 || out.shape[out.ndim - 1] != pv->out ||
       numel(out) != rows * pv->out)
     return kShape;
-  // what run_linears will ask of the scratch
+  // what run_linears will ask of the scratch, by the 256 x 128 tiles
+  // also where the register-decode GEMM takes the call, whose splits keep
+  // within the room beside the prepared rows (gemm_rd_plan)
   const bool gemm = rows > exl3::GEMV_ROWS_MAX && pv->f.gemm_rate();
   size_t slot_floats = 0, xp_bytes = 0, kpart_bytes = 0;
   if (gemm) {

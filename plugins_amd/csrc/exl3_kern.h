@@ -1844,11 +1844,13 @@ __global__ __launch_bounds__(GEMV_THREADS) void moe_gemv_kernel(
     run(std::integral_constant<int, PREP_PASSES>{});
 }
 
-// Grouped GEMM over routed work items (prefill-sized expert batches): the
-// specialised-wave GEMM with workgroup (column group cg, item) taking item
-// `blockIdx.y` = (expert e, up to 256 slots sorted[start ..]): activation
-// rows gathered by slot (x holds one prepared row per slot), expert e's
-// trellis words and svh, outputs scattered to the slots' rows.  No split k.
+// Grouped GEMM over a grouped linear's prompt rows, and over routed work items
+// where moe_gemm leaves them to it (banks that are not 16-byte aligned, few
+// workgroups over a short k): the specialised-wave GEMM with workgroup (column
+// group cg, item) taking item `blockIdx.y` = (expert e, up to 256 slots
+// sorted[start ..]): activation rows gathered by slot (x holds one prepared row
+// per slot), expert e's trellis words and svh, outputs scattered to the slots'
+// rows.  No split k.
 struct GemmGroup {
   const uint32_t *sorted;
   const MoeItem *items;

@@ -1056,7 +1056,8 @@ hipError_t launch_gemm_groups(const uint16_t *trellis, const Format &f, const ui
 //   1. route: one workgroup counts the (row, k) slots per expert, orders the
 //      slots by expert (within an expert in any order: every slot's
 //      arithmetic is independent of its position) and emits work items of
-//      up to 16 slots of one expert;
+//      up to 4 slots of one expert (of 64, 128 or 256 where moe_gemm takes a
+//      grouped GEMM, which then stands for the GEMVs);
 //   2. grouped GEMV, gate and up in one launch: each work item is the GEMV
 //      workgroup above over its expert's packed weights for its slots, the
 //      prepare (x[row] * suh[e]) fused, split-K with the fused finish,
