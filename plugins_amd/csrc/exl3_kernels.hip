@@ -1241,7 +1241,8 @@ void launch_moe_mid(const uint16_t *g, const uint16_t *u, const uint32_t *inds, 
 // columns a thread, U slots' loads in flight before their sums (1024 rows x top
 // 8 of 7168: 84 -> 24 us against a column a thread).  U: 2, 4 or 8, the least
 // that holds topk -- the rest of a wider pass is only more instructions (top 2 of
-// 512 columns, 1 row 2.84 us at U = 8, 2.00 at 2; of 4096, 16 rows 3.64 and 3.04).  wide: y is 16-byte aligned.
+// 512 columns, 1 row 2.84 us at U = 8, 2.00 at 2; of 4096, 16 rows 3.64 and
+// 3.04).  wide: y is 16-byte aligned.
 template <int U>
 __global__ __launch_bounds__(128) void moe_combine_kernel(const uint16_t *__restrict__ d,
                                                           const uint32_t *__restrict__ inds,
@@ -1541,11 +1542,11 @@ constexpr int MOE_PREFILL_SLOTS_PER_EXPERT = 32;
 // 512 at 8 0.80, 16 of 2048 x 512 at 8 0.97, 8 of 4096 x 1024 at 12 0.85, 12 of
 // 2048 x 256 at 17 0.72, 8 of 2048 x 512 at 17 0.80; under it 128 of 512 x 128 at
 // 4 1.10, 32 of 1024 x 128 at 8 1.11, 16 of 7168 x 512 at 8 1.22, 8 of 1024 x 128
-// at 31 1.43.  At 7 and 8 bits the GEMM's word loads weigh more (32 of 4096 x 1024
-// at 4 / 6 / 8 slots 1.23 / 1.04 / 0.88).
+// at 31 1.43.  At 7 and 8 bits the GEMM is the slower for longer (32 of 4096 x
+// 1024 at 4 / 6 / 8 slots 1.23 / 1.04 / 0.88), at the other rates alike.
 //
 // From 32 on the 256-slot GEMM is the other one (0.42-0.95 at 32 and 48 slots).
-// In few workgroups over a short k the finish and the items' second round weigh:
+// In few workgroups over a short k its larger tiles win from 64 slots on:
 // 8 experts of 512 x 256 at 64 / 96 / 128 / 200 / 300 slots 1.02 / 1.13 / 1.14 /
 // 1.01 / 0.95, 2 of 1024 x 512 0.93 / 1.07 / 1.15 / 1.03 / 0.97; 2 of 4096 x 2048
 // at 128 slots 0.95-1.01, at 8 bits 1.14.

@@ -255,7 +255,7 @@ def test_config3_routed_prefill_every_row(deepseek, tokens, path):
     """Every row against the float64 restatement, eight rows spread over the
     batch against the oracle.  At 1024 tokens (32 slots per expert on
     average) the experts' slots go through the grouped GEMM in items of up
-    to 256 slots."""
+    to 64 slots."""
     _, dev, _, _ = deepseek
     assert X.swiglu_path(dev[0], dev[1], dev[2], tokens, TOPK) == path
     sample = np.unique(np.linspace(0, tokens - 1, 8).astype(int))

@@ -437,8 +437,8 @@ def test_swiglu_clamp_keeps_nan(rows, which):
 @pytest.mark.parametrize("E,topk,rows,limit", [(4, 2, 128, 0), (2, 1, 600, 0), (3, 2, 200, 7)])
 def test_swiglu_routed_prefill_sizes(E, topk, rows, limit):
     # prefill-sized expert batches (32+ slots per expert on average, an
-    # expert past 256 slots): the grouped GEMM over routed items of <= 256
-    # slots, against the oracle's composition
+    # expert past 256 slots): the grouped GEMMs over routed items of <= 256
+    # and (300 an expert) <= 128 slots, against the oracle's composition
     rng = np.random.default_rng(E * 1000 + rows + limit)
     hidden, inter, n = 512, 256, 48
     g_np, g, g_keep = _bank(rng, E, hidden, inter, n)
