@@ -141,3 +141,29 @@ def test_rule_of_linears_that_share_rows(rows, apart):
     x = torch.from_numpy(S.activations(rng, rows, 1024)).to(DEV)
     ys = X.matmul_shared([lin.weight for lin in lins], x)
     assert all(torch.equal(y, lin(x)) for y, lin in zip(ys, lins)) == apart
+
+
+def test_unaligned_inputs():
+    """Rows and scales off their 16-byte boundaries: the prepare's narrower
+    accesses, in a shared call and in an MLP (whose SwiGLU then runs apart from
+    down's prepare), the same values."""
+    rng = np.random.default_rng(85)
+
+    def odd(a):
+        buf = torch.empty(a.numel() + 1, dtype=a.dtype, device=DEV)[1:]
+        buf.copy_(a.reshape(-1))
+        return buf.view(a.shape)
+
+    def pair(in_f, out_f):
+        t, u, v = S.linear(rng, in_f, out_f, 64)
+        t, u, v = (torch.from_numpy(a.view(k)).to(DEV)
+                   for a, k in ((t, np.int16), (u, np.float16), (v, np.float16)))
+        return X.wrap(t, u, v), X.wrap(t, odd(u), odd(v))
+
+    (g, go), (u, uo), (d, do) = pair(512, 640), pair(512, 640), pair(640, 512)
+    for dtype in (torch.float16, torch.bfloat16, torch.float32):
+        x = torch.from_numpy(S.activations(rng, 70, 512)).to(DEV).to(dtype)
+        xo = odd(x)
+        for a, b in zip(X.matmul_shared([g, u], x), X.matmul_shared([go, uo], xo)):
+            assert torch.equal(a, b)
+        assert torch.equal(X.swiglu(g, u, d, x), X.swiglu(go, uo, do, xo))
